@@ -89,6 +89,23 @@ int mm_route(const int32_t* selected, int64_t num_routes, int32_t top_k,
              void* workspace, size_t workspace_bytes, mm_stream_t stream);
 
 /*
+ * mm_route that also writes the M-tile lists of the row GEMMs (the expert's
+ * rows cut into tiles of at most 128 and of at most 256 rows) into `tiles`
+ * (mm_tile_lists_size(num_routes, num_experts) bytes, 16-byte aligned), so
+ * that the GEMMs of the pass, forward and backward, share them
+ * (mm_fc1_swiglu_tiles, mm_grouped_gemm_tiles) instead of building a list
+ * per launch. No counterpart in the reference.
+ */
+size_t mm_tile_lists_size(int64_t max_rows, int32_t num_experts);
+
+int mm_route_tiles(const int32_t* selected, int64_t num_routes, int32_t top_k,
+                   int32_t num_experts, const float* routing_weights,
+                   int32_t* counts, int32_t* offsets, int32_t* send_route,
+                   int32_t* send_token, int32_t* route_to_send,
+                   float* weight_perm, void* tiles, size_t tiles_bytes,
+                   void* workspace, size_t workspace_bytes, mm_stream_t stream);
+
+/*
  * mm_route without a workspace argument: the per-unit count table lives in
  * a library-owned device array of mm_route_noalloc_scratch_bytes() bytes
  * (4 MiB) per GPU, kept until the process ends. No counterpart in the
@@ -150,6 +167,19 @@ int mm_fc1_swiglu(const uint16_t* x, int64_t ldx, const int32_t* send_token,
                   void* workspace, size_t workspace_bytes, mm_stream_t stream);
 
 /*
+ * mm_fc1_swiglu on the tile lists mm_route_tiles wrote for the same offsets,
+ * max_rows (= its num_routes) and num_experts.
+ */
+int mm_fc1_swiglu_tiles(const uint16_t* x, int64_t ldx, const int32_t* send_token,
+                        const uint16_t* w1, const int32_t* offsets,
+                        const float* weight_perm, int32_t num_experts,
+                        int64_t max_rows, int32_t hidden, int32_t inter,
+                        int32_t act_kind, float situ_beta, float situ_linear_beta,
+                        float clamp_limit, uint16_t* act, void* fc1_out,
+                        int32_t fc1_format, float* fc1_scale,
+                        const void* tiles, size_t tiles_bytes, mm_stream_t stream);
+
+/*
  * Generic grouped "row" GEMM over expert-major rows:
  *   c[i, n] = sum_k a[row(i), k] * B_e(k, n),  e = expert of row i
  *   B_e(k, n) = b[e*b_se + n*b_sn + k*b_sk]   (one of b_sn, b_sk must be 1)
@@ -165,6 +195,14 @@ int mm_grouped_gemm(const uint16_t* a, int64_t lda, const int32_t* a_rows,
                     int64_t max_rows, int32_t n, int32_t k, uint16_t* c,
                     int64_t ldc, void* workspace, size_t workspace_bytes,
                     mm_stream_t stream);
+
+/* mm_grouped_gemm on the tile lists of mm_route_tiles (as mm_fc1_swiglu_tiles). */
+int mm_grouped_gemm_tiles(const uint16_t* a, int64_t lda, const int32_t* a_rows,
+                          const uint16_t* b, int64_t b_se, int64_t b_sn, int64_t b_sk,
+                          const int32_t* offsets, int32_t num_experts,
+                          int64_t max_rows, int32_t n, int32_t k, uint16_t* c,
+                          int64_t ldc, const void* tiles, size_t tiles_bytes,
+                          mm_stream_t stream);
 
 /*
  * Grouped weight-gradient GEMM with ragged K (the expert's rows):

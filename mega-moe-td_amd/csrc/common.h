@@ -29,6 +29,40 @@ static inline hipStream_t mm_hip_stream(mm_stream_t s) { return reinterpret_cast
 
 static inline size_t mm_align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+// ---------------------------------------------------------------- tile lists
+// M tiles of the row GEMMs: expert e's rows [offsets[e], offsets[e + 1]) cut
+// into tiles of at most BM rows, in expert order.
+struct TileList {
+  int32_t count;  // number of M tiles
+  int32_t pad[3];
+  int4 tiles[1];  // (expert, first row, end row, 0) per M tile
+};
+
+// Most M tiles of `max_rows` rows over E experts: sum ceil(c_e / BM) over the
+// at most min(E, max_rows) experts that hold rows.
+static inline int64_t mm_max_m_tiles(int64_t max_rows, int E, int BM) {
+  return max_rows / BM + (max_rows < E ? max_rows : E);
+}
+
+static inline size_t mm_tile_list_bytes(int64_t max_rows, int E, int BM) {
+  return mm_align_up(sizeof(TileList) + sizeof(int4) * static_cast<size_t>(mm_max_m_tiles(max_rows, E, BM)), 256);
+}
+
+// The two tile heights the row GEMMs use, in one buffer: the 128-row list,
+// then the 256-row list.
+static inline size_t mm_tile_lists_bytes(int64_t max_rows, int E) {
+  return mm_tile_list_bytes(max_rows, E, 128) + mm_tile_list_bytes(max_rows, E, 256);
+}
+
+static inline TileList* mm_tile_list_of(void* lists, int64_t max_rows, int E, int BM) {
+  char* p = static_cast<char*>(lists);
+  return reinterpret_cast<TileList*>(BM == 128 ? p : p + mm_tile_list_bytes(max_rows, E, 128));
+}
+
+// Fills one tile list from offsets (grouped_gemm.hip); the routing kernels
+// write both lists themselves up to their LDS bound.
+int mm_build_tiles(const int32_t* offsets, int E, int BM, TileList* tl, hipStream_t s);
+
 // ---------------------------------------------------------------- streaming loads
 // 16- / 8-byte loads of data read exactly once (gathered rows of the combine
 // and of the gated-activation backward): the non-temporal hint keeps them

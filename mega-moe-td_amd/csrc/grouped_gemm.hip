@@ -51,12 +51,6 @@ constexpr int BK = 64;
 constexpr int GROUP_M = 8;
 constexpr int kXcds = 8;
 
-struct TileList {
-  int32_t count;  // number of M tiles
-  int32_t pad[3];
-  int4 tiles[1];  // (expert, first row, end row, 0) per M tile
-};
-
 __global__ __launch_bounds__(1024) void build_tiles_kernel(const int32_t* __restrict__ offsets, int E, int BM,
                                                            TileList* __restrict__ tl) {
   __shared__ int part[1024];
@@ -1367,19 +1361,6 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
 }
 
 // ------------------------------------------------------------------ host side
-constexpr int kMinBM = 128;  // smallest M tile: sizes the tile list
-
-int64_t max_m_tiles(int64_t max_rows, int E, int BM) { return (max_rows + BM - 1) / BM + E; }
-
-size_t tile_list_bytes(int64_t max_rows, int E) {
-  return mm_align_up(sizeof(TileList) + sizeof(int4) * static_cast<size_t>(max_m_tiles(max_rows, E, kMinBM)), 256);
-}
-
-int launch_tiles(const int32_t* offsets, int E, int BM, void* ws, hipStream_t s) {
-  build_tiles_kernel<<<1, 1024, 0, s>>>(offsets, E, BM, static_cast<TileList*>(ws));
-  return mm_check_launch("build_tiles");
-}
-
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Row-GEMM tile choice: 256x256 when experts average at least 96 rows,
@@ -1405,7 +1386,7 @@ RowsCfg pick_rows_cfg(int64_t max_rows, int E, int n) {
 
 template <int BM, int BN, int BK_, int NST, int BLAYOUT, int EPI, int NT = kThreads, bool REG = false, int BPOL = 0>
 void launch_rows_cfg(const RowsArgs& p, int64_t max_rows, int E, hipStream_t s) {
-  const int64_t mm = max_m_tiles(max_rows, E, BM);
+  const int64_t mm = mm_max_m_tiles(max_rows, E, BM);
   const int64_t g = p.xcd_mod ? (mm + kXcds - 1) / kXcds * kXcds * (p.n / BN) : mm * (p.n / BN);
   const int grid = static_cast<int>((g + kXcds - 1) / kXcds * kXcds);
   if constexpr (EPI == EPI_GATED) {  // activation specialised at compile time
@@ -1487,18 +1468,30 @@ bool wgrad_reg(int64_t max_rows, int E) {
 }
 bool wgrad_small_k(int64_t max_rows, int E) { return max_rows <= kSmallKRows * static_cast<int64_t>(E); }
 
+// The M-tile list of a row GEMM: the lists mm_route_tiles wrote (lists), or
+// one made here from offsets (workspace).
+struct TileSource {
+  const void* lists;
+  void* workspace;
+  size_t bytes;
+};
+
 template <int BLAYOUT, int EPI>
-int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, void* ws, hipStream_t s,
+int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const TileSource& ts, hipStream_t s,
              const char* what) {
   const RowsCfg c = pick_rows_cfg(max_rows, E, p.n);
   // the largest grid any tile configuration launches (128-row M tiles padded
   // to a multiple of 8, 128-wide N tiles) must fit a 32-bit grid size
-  if ((max_m_tiles(max_rows, E, 128) + kXcds - 1) / kXcds * kXcds * (p.n / 128) >= (int64_t(1) << 31)) {
+  if ((mm_max_m_tiles(max_rows, E, 128) + kXcds - 1) / kXcds * kXcds * (p.n / 128) >= (int64_t(1) << 31)) {
     mm_set_error("%s: too many tiles for one launch", what);
     return MM_E_ARG;
   }
-  if (int rc = launch_tiles(offsets, E, c.bm, ws, s)) return rc;
-  p.tl = static_cast<const TileList*>(ws);
+  if (ts.lists) {
+    p.tl = mm_tile_list_of(const_cast<void*>(ts.lists), max_rows, E, c.bm);
+  } else {
+    if (int rc = mm_build_tiles(offsets, E, c.bm, static_cast<TileList*>(ts.workspace), s)) return rc;
+    p.tl = static_cast<const TileList*>(ts.workspace);
+  }
   // 128-row tiles (experts averaging < 256 rows, weight-streaming): one
   // expert's N tiles run together, so its gathered A panel stays in L2
   // (Kimi-scale: -5% layer time against 8-deep groups)
@@ -1559,30 +1552,38 @@ int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, void* 
 
 }  // namespace
 
-extern "C" size_t mm_gemm_workspace_bytes(int64_t max_rows, int32_t num_experts) {
-  return tile_list_bytes(max_rows, num_experts);
+int mm_build_tiles(const int32_t* offsets, int E, int BM, TileList* tl, hipStream_t s) {
+  build_tiles_kernel<<<1, 1024, 0, s>>>(offsets, E, BM, tl);
+  return mm_check_launch("build_tiles");
 }
 
-extern "C" int mm_fc1_swiglu(const uint16_t* x, int64_t ldx, const int32_t* send_token, const uint16_t* w1,
-                             const int32_t* offsets, const float* weight_perm, int32_t num_experts,
-                             int64_t max_rows, int32_t hidden, int32_t inter, int32_t act_kind, float situ_beta,
-                             float situ_linear_beta, float clamp_limit, uint16_t* act, void* fc1_out,
-                             int32_t fc1_format, float* fc1_scale, void* workspace, size_t workspace_bytes,
-                             mm_stream_t stream) {
-  MM_CHECK_ARG(x && w1 && offsets && weight_perm && act, "mm_fc1_swiglu: null pointer");
-  MM_CHECK_ARG(num_experts > 0 && max_rows >= 0 && max_rows < (int64_t(1) << 31), "mm_fc1_swiglu: bad sizes");
-  MM_CHECK_ARG(hidden > 0 && hidden % BK == 0, "mm_fc1_swiglu: hidden must be a multiple of %d", BK);
-  MM_CHECK_ARG(inter > 0 && inter % 64 == 0, "mm_fc1_swiglu: inter must be a multiple of 64");
-  MM_CHECK_ARG(ldx % 8 == 0 && al16(x) && al16(w1), "mm_fc1_swiglu: 16-byte alignment required");
-  MM_CHECK_ARG(act_kind >= 0 && act_kind <= 2, "mm_fc1_swiglu: bad act_kind");
-  MM_CHECK_ARG(fc1_format >= MM_FC1_BF16 && fc1_format <= MM_FC1_FP8, "mm_fc1_swiglu: bad fc1_format");
-  MM_CHECK_ARG(!fc1_out || fc1_format != MM_FC1_FP8 || (fc1_scale && inter % MM_FC1_SCALE_GROUP == 0),
-               "mm_fc1_swiglu: FP8 fc1_out needs fc1_scale and inter %% %d == 0", MM_FC1_SCALE_GROUP);
-  MM_CHECK_ARG(!fc1_out || (reinterpret_cast<uintptr_t>(fc1_out) & 7u) == 0, "mm_fc1_swiglu: fc1_out alignment");
-  if (!workspace || workspace_bytes < tile_list_bytes(max_rows, num_experts)) {
-    mm_set_error("mm_fc1_swiglu: workspace too small");
+namespace {
+
+int check_tile_source(const TileSource& ts, int64_t max_rows, int E, const char* what) {
+  const size_t need = ts.lists ? mm_tile_lists_bytes(max_rows, E) : mm_tile_list_bytes(max_rows, E, 128);
+  if ((!ts.lists && !ts.workspace) || ts.bytes < need) {
+    mm_set_error("%s: %s too small", what, ts.lists ? "tile lists" : "workspace");
     return MM_E_WS;
   }
+  return MM_OK;
+}
+
+int fc1_swiglu(const uint16_t* x, int64_t ldx, const int32_t* send_token, const uint16_t* w1,
+               const int32_t* offsets, const float* weight_perm, int32_t num_experts, int64_t max_rows,
+               int32_t hidden, int32_t inter, int32_t act_kind, float situ_beta, float situ_linear_beta,
+               float clamp_limit, uint16_t* act, void* fc1_out, int32_t fc1_format, float* fc1_scale,
+               TileSource ts, mm_stream_t stream, const char* what) {
+  MM_CHECK_ARG(x && w1 && offsets && weight_perm && act, "%s: null pointer", what);
+  MM_CHECK_ARG(num_experts > 0 && max_rows >= 0 && max_rows < (int64_t(1) << 31), "%s: bad sizes", what);
+  MM_CHECK_ARG(hidden > 0 && hidden % BK == 0, "%s: hidden must be a multiple of %d", what, BK);
+  MM_CHECK_ARG(inter > 0 && inter % 64 == 0, "%s: inter must be a multiple of 64", what);
+  MM_CHECK_ARG(ldx % 8 == 0 && al16(x) && al16(w1), "%s: 16-byte alignment required", what);
+  MM_CHECK_ARG(act_kind >= 0 && act_kind <= 2, "%s: bad act_kind", what);
+  MM_CHECK_ARG(fc1_format >= MM_FC1_BF16 && fc1_format <= MM_FC1_FP8, "%s: bad fc1_format", what);
+  MM_CHECK_ARG(!fc1_out || fc1_format != MM_FC1_FP8 || (fc1_scale && inter % MM_FC1_SCALE_GROUP == 0),
+               "%s: FP8 fc1_out needs fc1_scale and inter %% %d == 0", what, MM_FC1_SCALE_GROUP);
+  MM_CHECK_ARG(!fc1_out || (reinterpret_cast<uintptr_t>(fc1_out) & 7u) == 0, "%s: fc1_out alignment", what);
+  if (int rc = check_tile_source(ts, max_rows, num_experts, what)) return rc;
   if (max_rows == 0) return MM_OK;
   RowsArgs p{};
   p.a = reinterpret_cast<const bf16*>(x);
@@ -1605,26 +1606,22 @@ extern "C" int mm_fc1_swiglu(const uint16_t* x, int64_t ldx, const int32_t* send
   p.beta = situ_beta;
   p.lbeta = situ_linear_beta;
   p.clamp = clamp_limit;
-  return run_rows<B_NCONTIG, EPI_GATED>(p, offsets, max_rows, num_experts, workspace, mm_hip_stream(stream),
-                                        "mm_fc1_swiglu");
+  return run_rows<B_NCONTIG, EPI_GATED>(p, offsets, max_rows, num_experts, ts, mm_hip_stream(stream), what);
 }
 
-extern "C" int mm_grouped_gemm(const uint16_t* a, int64_t lda, const int32_t* a_rows, const uint16_t* b,
-                               int64_t b_se, int64_t b_sn, int64_t b_sk, const int32_t* offsets,
-                               int32_t num_experts, int64_t max_rows, int32_t n, int32_t k, uint16_t* c,
-                               int64_t ldc, void* workspace, size_t workspace_bytes, mm_stream_t stream) {
-  MM_CHECK_ARG(a && b && offsets && c, "mm_grouped_gemm: null pointer");
-  MM_CHECK_ARG(num_experts > 0 && max_rows >= 0 && max_rows < (int64_t(1) << 31), "mm_grouped_gemm: bad sizes");
-  MM_CHECK_ARG(n > 0 && n % 128 == 0, "mm_grouped_gemm: n must be a multiple of 128");
-  MM_CHECK_ARG(k > 0 && k % BK == 0, "mm_grouped_gemm: k must be a multiple of %d", BK);
-  MM_CHECK_ARG(b_sn == 1 || b_sk == 1, "mm_grouped_gemm: B must be contiguous along N or K");
+int grouped_gemm(const uint16_t* a, int64_t lda, const int32_t* a_rows, const uint16_t* b, int64_t b_se,
+                 int64_t b_sn, int64_t b_sk, const int32_t* offsets, int32_t num_experts, int64_t max_rows,
+                 int32_t n, int32_t k, uint16_t* c, int64_t ldc, TileSource ts, mm_stream_t stream,
+                 const char* what) {
+  MM_CHECK_ARG(a && b && offsets && c, "%s: null pointer", what);
+  MM_CHECK_ARG(num_experts > 0 && max_rows >= 0 && max_rows < (int64_t(1) << 31), "%s: bad sizes", what);
+  MM_CHECK_ARG(n > 0 && n % 128 == 0, "%s: n must be a multiple of 128", what);
+  MM_CHECK_ARG(k > 0 && k % BK == 0, "%s: k must be a multiple of %d", what, BK);
+  MM_CHECK_ARG(b_sn == 1 || b_sk == 1, "%s: B must be contiguous along N or K", what);
   MM_CHECK_ARG(lda % 8 == 0 && al16(a) && al16(b) && (b_sn == 1 ? b_sk % 8 == 0 : b_sn % 8 == 0) &&
                    b_se % 8 == 0,
-               "mm_grouped_gemm: 16-byte alignment required");
-  if (!workspace || workspace_bytes < tile_list_bytes(max_rows, num_experts)) {
-    mm_set_error("mm_grouped_gemm: workspace too small");
-    return MM_E_WS;
-  }
+               "%s: 16-byte alignment required", what);
+  if (int rc = check_tile_source(ts, max_rows, num_experts, what)) return rc;
   if (max_rows == 0) return MM_OK;
   RowsArgs p{};
   p.a = reinterpret_cast<const bf16*>(a);
@@ -1639,8 +1636,54 @@ extern "C" int mm_grouped_gemm(const uint16_t* a, int64_t lda, const int32_t* a_
   p.c = reinterpret_cast<bf16*>(c);
   p.ldc = ldc;
   hipStream_t s = mm_hip_stream(stream);
-  if (b_sk == 1) return run_rows<B_KCONTIG, EPI_STORE>(p, offsets, max_rows, num_experts, workspace, s, "mm_grouped_gemm");
-  return run_rows<B_NCONTIG, EPI_STORE>(p, offsets, max_rows, num_experts, workspace, s, "mm_grouped_gemm");
+  if (b_sk == 1) return run_rows<B_KCONTIG, EPI_STORE>(p, offsets, max_rows, num_experts, ts, s, what);
+  return run_rows<B_NCONTIG, EPI_STORE>(p, offsets, max_rows, num_experts, ts, s, what);
+}
+
+}  // namespace
+
+extern "C" int mm_fc1_swiglu(const uint16_t* x, int64_t ldx, const int32_t* send_token, const uint16_t* w1,
+                             const int32_t* offsets, const float* weight_perm, int32_t num_experts,
+                             int64_t max_rows, int32_t hidden, int32_t inter, int32_t act_kind, float situ_beta,
+                             float situ_linear_beta, float clamp_limit, uint16_t* act, void* fc1_out,
+                             int32_t fc1_format, float* fc1_scale, void* workspace, size_t workspace_bytes,
+                             mm_stream_t stream) {
+  return fc1_swiglu(x, ldx, send_token, w1, offsets, weight_perm, num_experts, max_rows, hidden, inter, act_kind,
+                    situ_beta, situ_linear_beta, clamp_limit, act, fc1_out, fc1_format, fc1_scale,
+                    TileSource{nullptr, workspace, workspace_bytes}, stream, "mm_fc1_swiglu");
+}
+
+extern "C" int mm_fc1_swiglu_tiles(const uint16_t* x, int64_t ldx, const int32_t* send_token, const uint16_t* w1,
+                                   const int32_t* offsets, const float* weight_perm, int32_t num_experts,
+                                   int64_t max_rows, int32_t hidden, int32_t inter, int32_t act_kind,
+                                   float situ_beta, float situ_linear_beta, float clamp_limit, uint16_t* act,
+                                   void* fc1_out, int32_t fc1_format, float* fc1_scale, const void* tiles,
+                                   size_t tiles_bytes, mm_stream_t stream) {
+  MM_CHECK_ARG(tiles, "mm_fc1_swiglu_tiles: null pointer");
+  return fc1_swiglu(x, ldx, send_token, w1, offsets, weight_perm, num_experts, max_rows, hidden, inter, act_kind,
+                    situ_beta, situ_linear_beta, clamp_limit, act, fc1_out, fc1_format, fc1_scale,
+                    TileSource{tiles, nullptr, tiles_bytes}, stream, "mm_fc1_swiglu_tiles");
+}
+
+extern "C" int mm_grouped_gemm(const uint16_t* a, int64_t lda, const int32_t* a_rows, const uint16_t* b,
+                               int64_t b_se, int64_t b_sn, int64_t b_sk, const int32_t* offsets,
+                               int32_t num_experts, int64_t max_rows, int32_t n, int32_t k, uint16_t* c,
+                               int64_t ldc, void* workspace, size_t workspace_bytes, mm_stream_t stream) {
+  return grouped_gemm(a, lda, a_rows, b, b_se, b_sn, b_sk, offsets, num_experts, max_rows, n, k, c, ldc,
+                      TileSource{nullptr, workspace, workspace_bytes}, stream, "mm_grouped_gemm");
+}
+
+extern "C" int mm_grouped_gemm_tiles(const uint16_t* a, int64_t lda, const int32_t* a_rows, const uint16_t* b,
+                                     int64_t b_se, int64_t b_sn, int64_t b_sk, const int32_t* offsets,
+                                     int32_t num_experts, int64_t max_rows, int32_t n, int32_t k, uint16_t* c,
+                                     int64_t ldc, const void* tiles, size_t tiles_bytes, mm_stream_t stream) {
+  MM_CHECK_ARG(tiles, "mm_grouped_gemm_tiles: null pointer");
+  return grouped_gemm(a, lda, a_rows, b, b_se, b_sn, b_sk, offsets, num_experts, max_rows, n, k, c, ldc,
+                      TileSource{tiles, nullptr, tiles_bytes}, stream, "mm_grouped_gemm_tiles");
+}
+
+extern "C" size_t mm_gemm_workspace_bytes(int64_t max_rows, int32_t num_experts) {
+  return mm_tile_list_bytes(max_rows, num_experts, 128);  // 128 rows: the longer of the two lists
 }
 
 // Every weight-gradient kernel gathers its rows in place: no workspace.

@@ -7,20 +7,27 @@
 // core-minor prefix, then an order-preserving scatter) and
 // kernels/fc2_combine.py:508-529 inverts it (route_to_send, -1 for drops).
 //
-// MI355X design: three small launches, no global atomics, no host sync.
-// Up to 1024 experts the scatter runs four wavefronts per unit; above that
-// (up to 32768, bounded by LDS) one wavefront per unit, whose ballot match
-// masks alone give the stable rank (the reference's lower-bound path for
-// large bin counts, runtime/routing.py:246-416, serves the same range).
-//   1. route_count   one workgroup per chunk of ROUTE_CHUNK consecutive routes
-//                    builds an LDS histogram -> unit_counts[unit][expert].
-//   2. route_scan    one workgroup turns unit_counts into absolute start rows
-//                    (expert-major, unit-minor), counts[] and offsets[E+1].
-//   3. route_scatter each workgroup replays its chunk 256 routes at a time; a
-//                    route's rank among equal experts inside a wavefront comes
-//                    from ballot "match" masks, across the four wavefronts from
-//                    tagged LDS counters, so the scatter is stable without a
-//                    sort and writes every table exactly once.
+// MI355X design: no global atomics, no host sync, no sort.
+// Up to 1024 experts (route_fused_kernel): a unit is 2048 consecutive routes
+// and one 16-wavefront workgroup. A workgroup needs, per expert, the routes in
+// earlier units and in all units; mostly it counts them itself from the ids
+// (L2-resident), so routing is ONE launch; else a first launch writes
+// unit_counts[unit][expert] and every workgroup sums the table (see
+// recount_routes). A block scan over the experts then gives every expert's
+// first row, and each wavefront scatters its own 128 routes in order: a
+// route's rank among equal experts comes from ballot match masks, the running
+// counter per (wavefront, expert) sits in LDS, so the scatter is
+// stable and needs no workgroup barrier. The last workgroup also writes the
+// M-tile lists of the row GEMMs.
+// It is latency-bound. Three launches (count, scan, scatter) without tile
+// lists measured, against this form with them (graph replay, us): 8 routes
+// over 128 experts 10.1 -> 5.9, 4084 over 60 17.0 -> 8.0, 32768 over 32 19.6
+// -> 11.2, 65536 over 896 27.2 -> 15.9; each tile list built by itself was
+// another 3 to 7 us launch, two per forward and two per backward.
+// Above 1024 experts (up to 32768, bounded by LDS) count, scan and a
+// one-wavefront scatter per unit remain three launches (the reference's
+// lower-bound path for large bin counts, runtime/routing.py:246-416, serves
+// the same range).
 #include <mutex>
 
 #include "common.h"
@@ -28,10 +35,11 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / 64;
-constexpr int kIters = 8;                       // 256-route steps per unit
-constexpr int kChunk = kThreads * kIters;       // routes per unit
-constexpr int kMaxExperts4 = 1024;              // LDS bound of the 4-wave route_scatter (36 KiB)
+constexpr int kChunk = 2048;                    // routes per unit
+constexpr int kFusedThreads = 1024;
+constexpr int kFusedWaves = kFusedThreads / 64;
+constexpr int kSeg = kChunk / kFusedWaves;      // consecutive routes per wavefront of a unit
+constexpr int kFusedExperts = 1024;             // LDS bound of route_fused_kernel (72 KiB)
 constexpr int kMaxExperts = 32768;              // LDS bound of the 1-wave scatter (128 KiB) and the scan
 
 __device__ __forceinline__ bool route_valid(int e, int E) { return e >= 0 && e < E; }
@@ -111,67 +119,150 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int32_t* __restrict__ 
   }
 }
 
-__global__ __launch_bounds__(kThreads) void route_scatter_kernel(
-    const int32_t* __restrict__ sel, int64_t R, int top_k, int E, int nbits,
-    const int32_t* __restrict__ unit_base, const float* __restrict__ rw,
-    int32_t* __restrict__ send_route, int32_t* __restrict__ send_token,
-    int32_t* __restrict__ route_to_send, float* __restrict__ weight_perm) {
-  extern __shared__ int lds[];
-  int* run = lds;                 // [E]   next free row of each expert
-  int* wcnt = run + E;            // [kWaves][E] routes of expert e in wave w (this step)
-  int* wtag = wcnt + kWaves * E;  // [kWaves][E] step id that wrote wcnt
-  const int u = blockIdx.x;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  for (int e = threadIdx.x; e < E; e += kThreads) {
-    run[e] = unit_base[static_cast<int64_t>(u) * E + e];
+// Inclusive scan of v over the 1024 threads of a workgroup (wave shuffles,
+// then the 16 wave totals); part is LDS scratch of kFusedWaves entries.
+__device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t* part) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) wtag[w * E + e] = -1;
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint64_t o = __shfl_up(v, off);
+    if (lane >= off) v += o;
+  }
+  if (lane == 63) part[wave] = v;
+  __syncthreads();
+  uint64_t base = 0;
+#pragma unroll
+  for (int w = 0; w < kFusedWaves; ++w) base += w < wave ? part[w] : 0;
+  __syncthreads();
+  return v + base;
+}
+
+// One workgroup per unit, E <= kFusedExperts. unit_counts: null (count all
+// routes here) or the [nunits][E] table of route_count_kernel.
+__global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
+    const int32_t* __restrict__ sel, int64_t R, int top_k, int E, int nbits, int nunits,
+    const int32_t* __restrict__ unit_counts, const float* __restrict__ rw, int32_t* __restrict__ counts,
+    int32_t* __restrict__ offsets, int32_t* __restrict__ send_route, int32_t* __restrict__ send_token,
+    int32_t* __restrict__ route_to_send, float* __restrict__ weight_perm, TileList* __restrict__ tl128,
+    TileList* __restrict__ tl256) {
+  __shared__ int seg[kFusedWaves * kFusedExperts];  // [wave][expert]: routes of the segment, then its next row
+  __shared__ int before[kFusedExperts], rest[kFusedExperts];  // routes in earlier / later units
+  __shared__ uint64_t part[kFusedWaves];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int u = blockIdx.x;
+  const int64_t start = static_cast<int64_t>(u) * kChunk;
+  const int64_t end = min(R, start + kChunk);
+  for (int i = tid; i < kFusedWaves * E; i += kFusedThreads) seg[i] = 0;
+  for (int e = tid; e < E; e += kFusedThreads) before[e] = rest[e] = 0;
+  __syncthreads();
+
+  // own unit: counts per wavefront segment (wave w owns routes start + w * kSeg ..)
+  constexpr int ITERS = kSeg / 64;
+  int key[ITERS];
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int64_t i = start + wave * kSeg + it * 64 + lane;
+    const int e = i < R ? sel[i] : -1;
+    key[it] = route_valid(e, E) ? e : E;
+    if (key[it] < E) atomicAdd(&seg[wave * E + key[it]], 1);
+  }
+  if (unit_counts) {
+    for (int i = tid; i < nunits * E; i += kFusedThreads) {
+      const int v = i / E, e = i - v * E;
+      const int c = unit_counts[i];
+      if (v != u && c) atomicAdd(v < u ? &before[e] : &rest[e], c);
+    }
+  } else {
+    auto count = [&](int64_t lo, int64_t hi, int* hist) {
+      int64_t i = lo + tid;
+      for (; i + 7 * kFusedThreads < hi; i += 8 * kFusedThreads) {
+        int e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = sel[i + j * kFusedThreads];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (route_valid(e[j], E)) atomicAdd(&hist[e[j]], 1);
+      }
+      for (; i < hi; i += kFusedThreads) {
+        const int e = sel[i];
+        if (route_valid(e, E)) atomicAdd(&hist[e], 1);
+      }
+    };
+    count(0, start, before);
+    count(end, R, rest);
   }
   __syncthreads();
+
+  // per expert: first row of every segment relative to the expert, then the
+  // expert's first row from a scan over the experts
+  int total = 0;
+  if (tid < E) {
+    int run = before[tid];
+#pragma unroll
+    for (int w = 0; w < kFusedWaves; ++w) {
+      const int c = seg[w * E + tid];
+      seg[w * E + tid] = run;
+      run += c;
+    }
+    total = run + rest[tid];
+  }
+  const int first = static_cast<int>(block_scan(static_cast<uint64_t>(total), part)) - total;
+  if (tid < E) {
+#pragma unroll
+    for (int w = 0; w < kFusedWaves; ++w) seg[w * E + tid] += first;
+    if (u == 0) {
+      counts[tid] = total;
+      offsets[tid] = first;
+      if (tid == E - 1) offsets[E] = first + total;
+    }
+  }
+  if (u == nunits - 1 && tl128) {
+    const uint64_t t128 = (total + 127) / 128, t256 = (total + 255) / 256;
+    const uint64_t t = block_scan(t128 | (t256 << 32), part);
+    if (tid < E) {
+      int n = static_cast<int>(t & 0xffffffffu) - static_cast<int>(t128);
+      for (int r = 0; r < total; r += 128) tl128->tiles[n++] = make_int4(tid, first + r, first + min(r + 128, total), 0);
+      n = static_cast<int>(t >> 32) - static_cast<int>(t256);
+      for (int r = 0; r < total; r += 256) tl256->tiles[n++] = make_int4(tid, first + r, first + min(r + 256, total), 0);
+    }
+    if (tid == kFusedThreads - 1) {
+      tl128->count = static_cast<int>(t & 0xffffffffu);
+      tl256->count = static_cast<int>(t >> 32);
+    }
+  }
+  __syncthreads();
+
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int64_t start = static_cast<int64_t>(u) * kChunk;
-  for (int it = 0; it < kIters; ++it) {
-    const int64_t i = start + static_cast<int64_t>(it) * kThreads + threadIdx.x;
-    const bool present = i < R;
-    int e = present ? sel[i] : -1;
-    const bool valid = present && route_valid(e, E);
-    const int key = valid ? e : E;  // E = "not routed"
-    // match mask: lanes of this wave holding the same key
-    uint64_t mask = __ballot(1);
+  int* next = seg + wave * E;  // this wavefront's counters: LDS operations of one wave stay in order
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it) {
+    const int64_t i = start + wave * kSeg + it * 64 + lane;
+    const bool present = i < R, valid = key[it] < E;
+    uint64_t mask = __ballot(1);  // lanes holding the same key
     for (int b = 0; b < nbits; ++b) {
-      const bool bit = (key >> b) & 1;
+      const bool bit = (key[it] >> b) & 1;
       const uint64_t m = __ballot(bit);
       mask &= bit ? m : ~m;
     }
-    const int rank_in_wave = __popcll(mask & lt_mask);
-    const int cnt_in_wave = __popcll(mask);
-    const bool leader = valid && rank_in_wave == 0;
-    if (leader) {
-      wcnt[wave * E + key] = cnt_in_wave;
-      wtag[wave * E + key] = it;
-    }
-    __syncthreads();
+    const int rank = __popcll(mask & lt_mask);
+    const int base = valid ? next[key[it]] : 0;
+    asm volatile("" ::: "memory");  // every lane reads its counter before a leader moves it
+    if (valid && rank == 0) next[key[it]] = base + __popcll(mask);
+    asm volatile("" ::: "memory");
     if (present) {
+      const int pos = valid ? base + rank : -1;
+      route_to_send[i] = pos;
       if (valid) {
-        int pos = run[key] + rank_in_wave;
-        for (int w = 0; w < wave; ++w)
-          if (wtag[w * E + key] == it) pos += wcnt[w * E + key];
         send_route[pos] = static_cast<int32_t>(i);
         send_token[pos] = static_cast<int32_t>(i / top_k);
-        route_to_send[i] = pos;
         if (weight_perm != nullptr) weight_perm[pos] = rw[i];
-      } else {
-        route_to_send[i] = -1;
       }
     }
-    __syncthreads();
-    if (leader) atomicAdd(&run[key], cnt_in_wave);
-    __syncthreads();
   }
 }
 
-// Scatter for large expert counts (E > kMaxExperts4): one wavefront per unit,
+// Scatter for large expert counts (E > kFusedExperts): one wavefront per unit,
 // so the stable rank of a route among equal experts comes from the ballot
 // match mask alone and LDS holds only the E running row counters.
 __global__ __launch_bounds__(64) void route_scatter_wave_kernel(
@@ -226,44 +317,56 @@ extern "C" size_t mm_route_workspace_bytes(int64_t num_routes, int32_t num_exper
 
 namespace {
 
+// Whether every unit counts the other units' routes itself instead of
+// summing a table that a first launch writes. Recounting costs each workgroup
+// R ids, the table its R / 2048 * E entries and a launch; measured (us,
+// recount / table): 65536 routes 14.3 / 13.1 over 128 experts and 15.9 / 23.9
+// over 896; 131072 routes over 32 experts 21.7 / 12.8. At 32768 routes and
+// below the launch alone costs more (11.2 over 32 experts, all of it).
+bool recount_routes(int64_t num_routes, int E) { return num_routes <= 32768 || E >= 512; }
+
 int route_launch(const int32_t* selected, int64_t num_routes, int32_t top_k, int32_t num_experts,
                  const float* routing_weights, int32_t* counts, int32_t* offsets, int32_t* send_route,
                  int32_t* send_token, int32_t* route_to_send, float* weight_perm, int32_t* unit_counts,
-                 hipStream_t s, const char* what) {
+                 void* tiles, hipStream_t s, const char* what) {
   const int E = num_experts;
   const int nunits = static_cast<int>((num_routes + kChunk - 1) / kChunk);
-  if (E > kMaxExperts4) {
-    // dynamic LDS above 64 KiB (up to 132 KiB at kMaxExperts); set once
-    static std::once_flag once;
-    std::call_once(once, [] {
-      const int bytes = (kMaxExperts + 1024) * static_cast<int>(sizeof(int));
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(route_count_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(route_scan_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(route_scatter_wave_kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    });
+  const int nbits = 32 - __builtin_clz(static_cast<unsigned>(E));
+  TileList* tl128 = tiles ? mm_tile_list_of(tiles, num_routes, E, 128) : nullptr;
+  TileList* tl256 = tiles ? mm_tile_list_of(tiles, num_routes, E, 256) : nullptr;
+  if (E <= kFusedExperts) {
+    const bool recount = recount_routes(num_routes, E);
+    if (!recount)
+      route_count_kernel<<<nunits, kThreads, E * sizeof(int), s>>>(selected, num_routes, E, nunits, unit_counts);
+    route_fused_kernel<<<nunits > 0 ? nunits : 1, kFusedThreads, 0, s>>>(
+        selected, num_routes, top_k, E, nbits, nunits > 0 ? nunits : 1, recount ? nullptr : unit_counts,
+        routing_weights, counts, offsets, send_route, send_token, route_to_send, weight_perm, tl128, tl256);
+    return mm_check_launch(what);
   }
-  if (nunits > 0) {
-    route_count_kernel<<<nunits, kThreads, E * sizeof(int), s>>>(selected, num_routes, E, nunits,
-                                                                 unit_counts);
-  }
+  // dynamic LDS above 64 KiB (up to 132 KiB at kMaxExperts); set once
+  static std::once_flag once;
+  std::call_once(once, [] {
+    const int bytes = (kMaxExperts + 1024) * static_cast<int>(sizeof(int));
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(route_count_kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(route_scan_kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(route_scatter_wave_kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  });
+  if (nunits > 0)
+    route_count_kernel<<<nunits, kThreads, E * sizeof(int), s>>>(selected, num_routes, E, nunits, unit_counts);
   route_scan_kernel<<<1, 1024, (E + 1024) * sizeof(int), s>>>(unit_counts, E, nunits, counts, offsets);
-  if (nunits > 0) {
-    const int nbits = 32 - __builtin_clz(static_cast<unsigned>(E));
-    if (E <= kMaxExperts4) {
-      const size_t lds = static_cast<size_t>(E) * (1 + 2 * kWaves) * sizeof(int);
-      route_scatter_kernel<<<nunits, kThreads, lds, s>>>(selected, num_routes, top_k, E, nbits, unit_counts,
-                                                         routing_weights, send_route, send_token,
-                                                         route_to_send, weight_perm);
-    } else {
-      route_scatter_wave_kernel<<<nunits, 64, static_cast<size_t>(E) * sizeof(int), s>>>(
-          selected, num_routes, top_k, E, nbits, unit_counts, routing_weights, send_route, send_token,
-          route_to_send, weight_perm);
-    }
+  if (nunits > 0)
+    route_scatter_wave_kernel<<<nunits, 64, static_cast<size_t>(E) * sizeof(int), s>>>(
+        selected, num_routes, top_k, E, nbits, unit_counts, routing_weights, send_route, send_token,
+        route_to_send, weight_perm);
+  if (int rc = mm_check_launch(what)) return rc;
+  if (tiles) {
+    if (int rc = mm_build_tiles(offsets, E, 128, tl128, s)) return rc;
+    return mm_build_tiles(offsets, E, 256, tl256, s);
   }
-  return mm_check_launch(what);
+  return MM_OK;
 }
 
 }  // namespace
@@ -290,8 +393,33 @@ extern "C" int mm_route(const int32_t* selected, int64_t num_routes, int32_t top
     return MM_E_WS;
   }
   return route_launch(selected, num_routes, top_k, num_experts, routing_weights, counts, offsets, send_route,
-                      send_token, route_to_send, weight_perm, static_cast<int32_t*>(workspace),
+                      send_token, route_to_send, weight_perm, static_cast<int32_t*>(workspace), nullptr,
                       mm_hip_stream(stream), "mm_route");
+}
+
+extern "C" size_t mm_tile_lists_size(int64_t max_rows, int32_t num_experts) {
+  return mm_tile_lists_bytes(max_rows, num_experts);
+}
+
+extern "C" int mm_route_tiles(const int32_t* selected, int64_t num_routes, int32_t top_k, int32_t num_experts,
+                              const float* routing_weights, int32_t* counts, int32_t* offsets,
+                              int32_t* send_route, int32_t* send_token, int32_t* route_to_send,
+                              float* weight_perm, void* tiles, size_t tiles_bytes, void* workspace,
+                              size_t workspace_bytes, mm_stream_t stream) {
+  MM_ROUTE_CHECK_ARGS("mm_route_tiles");
+  if (workspace_bytes < mm_route_workspace_bytes(num_routes, num_experts) || workspace == nullptr) {
+    mm_set_error("mm_route_tiles: workspace too small");
+    return MM_E_WS;
+  }
+  if (tiles == nullptr || (reinterpret_cast<uintptr_t>(tiles) & 15u) ||
+      tiles_bytes < mm_tile_lists_bytes(num_routes, num_experts)) {
+    mm_set_error("mm_route_tiles: tile lists need %zu bytes, 16-byte aligned",
+                 mm_tile_lists_bytes(num_routes, num_experts));
+    return MM_E_WS;
+  }
+  return route_launch(selected, num_routes, top_k, num_experts, routing_weights, counts, offsets, send_route,
+                      send_token, route_to_send, weight_perm, static_cast<int32_t*>(workspace), tiles,
+                      mm_hip_stream(stream), "mm_route_tiles");
 }
 
 // ---------------------------------------------------------------- no-allocation variant
@@ -352,5 +480,5 @@ extern "C" int mm_route_noalloc(const int32_t* selected, int64_t num_routes, int
   int32_t* ws = nullptr;
   if (int rc = scratch_for_current_device(&ws)) return rc;
   return route_launch(selected, num_routes, top_k, num_experts, routing_weights, counts, offsets, send_route,
-                      send_token, route_to_send, weight_perm, ws, mm_hip_stream(stream), "mm_route_noalloc");
+                      send_token, route_to_send, weight_perm, ws, nullptr, mm_hip_stream(stream), "mm_route_noalloc");
 }

@@ -33,6 +33,8 @@ SIGNATURES = {
     "mm_version": (ctypes.c_int, []),
     "mm_route_workspace_bytes": (_SZ, [_I64, _I32]),
     "mm_route": (ctypes.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
+    "mm_tile_lists_size": (_SZ, [_I64, _I32]),
+    "mm_route_tiles": (ctypes.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P, _SZ, _P]),
     "mm_route_noalloc_scratch_bytes": (_SZ, []),
     "mm_route_noalloc": (ctypes.c_int, [_P, _I64, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P]),
     "mm_permute": (ctypes.c_int, [_P, _I64, _P, _P, _I32, _I64, _I32, _P, _I64, _P]),
@@ -42,6 +44,10 @@ SIGNATURES = {
                                      _F32, _F32, _F32, _P, _P, _I32, _P, _P, _SZ, _P]),
     "mm_grouped_gemm": (ctypes.c_int, [_P, _I64, _P, _P, _I64, _I64, _I64, _P, _I32, _I64, _I32,
                                        _I32, _P, _I64, _P, _SZ, _P]),
+    "mm_fc1_swiglu_tiles": (ctypes.c_int, [_P, _I64, _P, _P, _P, _P, _I32, _I64, _I32, _I32, _I32,
+                                           _F32, _F32, _F32, _P, _P, _I32, _P, _P, _SZ, _P]),
+    "mm_grouped_gemm_tiles": (ctypes.c_int, [_P, _I64, _P, _P, _I64, _I64, _I64, _P, _I32, _I64, _I32,
+                                             _I32, _P, _I64, _P, _SZ, _P]),
     "mm_grouped_wgrad": (ctypes.c_int, [_P, _I64, _P, _P, _I64, _P, _P, _I32, _I64, _I32, _I32, _P, _P,
                                         _SZ, _P]),
     "mm_combine": (ctypes.c_int, [_P, _I64, _P, _I64, _I32, _I32, _P, _I64, _P]),

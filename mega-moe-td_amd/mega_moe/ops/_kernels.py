@@ -107,11 +107,12 @@ def fc1_format_of(t: torch.Tensor) -> str:
 
 
 def fc1_swiglu(x, send_token, w1, offsets, weight_perm, max_rows: int, activation: str, situ_beta: float,
-               situ_linear_beta, clamp_limit: float, save_fc1: bool, fc1_dtype: str = "bf16", pool=None):
+               situ_linear_beta, clamp_limit: float, save_fc1: bool, fc1_dtype: str = "bf16", pool=None, tiles=None):
     """FC1 grouped GEMM + weighted gated activation.
 
     Returns (act [rows, I] bf16, fc1_output [rows, 2I] in ``fc1_dtype`` | None,
-    fc1_scale [rows, 2I / 128] fp32 for fp8 | None).
+    fc1_scale [rows, 2I / 128] fp32 for fp8 | None). ``tiles``: the tile lists
+    routing wrote for these offsets and ``max_rows``; built here without them.
     """
     _check_bf16("x", x)
     _check_bf16("w1", w1)
@@ -129,9 +130,9 @@ def fc1_swiglu(x, send_token, w1, offsets, weight_perm, max_rows: int, activatio
         if inter % _lib.FC1_SCALE_GROUP:
             raise ValueError(f"fp8 fc1 save needs ffn % {_lib.FC1_SCALE_GROUP} == 0, got {inter}")
         fc1_scale = torch.empty(max_rows, two_inter // _lib.FC1_SCALE_GROUP, dtype=torch.float32, device=dev)
-    ws = _gemm_ws(dev, max_rows, num_experts, pool)
+    ws = tiles if tiles is not None else _gemm_ws(dev, max_rows, num_experts, pool)
     lbeta = float(situ_linear_beta) if situ_linear_beta is not None else 0.0
-    _lib.call("mm_fc1_swiglu", _lib.ptr(x), x.stride(0), _lib.ptr(send_token), _lib.ptr(w1), _lib.ptr(offsets),
+    _lib.call("mm_fc1_swiglu" if tiles is None else "mm_fc1_swiglu_tiles", _lib.ptr(x), x.stride(0), _lib.ptr(send_token), _lib.ptr(w1), _lib.ptr(offsets),
               _lib.ptr(weight_perm), num_experts, max_rows, hidden, inter, _lib.ACT_KINDS[activation],
               float(situ_beta), lbeta, float(clamp_limit), _lib.ptr(act), _lib.ptr(fc1_out),
               _lib.FC1_FORMATS[fc1_dtype], _lib.ptr(fc1_scale), _lib.ptr(ws), ws.numel(), _lib.stream_of(dev))
@@ -139,16 +140,18 @@ def fc1_swiglu(x, send_token, w1, offsets, weight_perm, max_rows: int, activatio
 
 
 def grouped_gemm(a, a_rows, b, b_se: int, b_sn: int, b_sk: int, offsets, max_rows: int, n: int, k: int,
-                 pool=None):
-    """c[i, :] = a[row(i), :] @ B_e for expert-major rows; B_e(k, n) = b[e*se + n*sn + k*sk]."""
+                 pool=None, tiles=None):
+    """c[i, :] = a[row(i), :] @ B_e for expert-major rows; B_e(k, n) = b[e*se + n*sn + k*sk].
+
+    ``tiles``: the tile lists routing wrote for these offsets and ``max_rows``."""
     _check_bf16("a", a)
     _check_bf16("b", b)
     if a.stride(1) != 1 or a.shape[1] != k:
         raise ValueError("grouped_gemm: a must be [*, K] with unit column stride")
     num_experts = offsets.numel() - 1
     c = torch.empty(max_rows, n, dtype=torch.bfloat16, device=a.device)
-    ws = _gemm_ws(a.device, max_rows, num_experts, pool)
-    _lib.call("mm_grouped_gemm", _lib.ptr(a), a.stride(0), _lib.ptr(a_rows), _lib.ptr(b), b_se, b_sn, b_sk,
+    ws = tiles if tiles is not None else _gemm_ws(a.device, max_rows, num_experts, pool)
+    _lib.call("mm_grouped_gemm" if tiles is None else "mm_grouped_gemm_tiles", _lib.ptr(a), a.stride(0), _lib.ptr(a_rows), _lib.ptr(b), b_se, b_sn, b_sk,
               _lib.ptr(offsets), num_experts, max_rows, n, k, _lib.ptr(c), c.stride(0), _lib.ptr(ws), ws.numel(),
               _lib.stream_of(a.device))
     return c

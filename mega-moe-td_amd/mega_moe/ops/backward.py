@@ -105,10 +105,12 @@ def moe_backward_triton(saved, dy, peer_mem=None, grad_transport=None, hidden_st
     tm.mark_pass()
     pool = saved.get("_workspaces")
     ws_rows = saved.get("_max_routes") or R
+    tiles = saved.get("_tiles")
     # step 1: FC2 dgrad, B_e(k=h, n=f) = down[e, h, f]
     tm.begin("fc2_dgrad")
     se, sh, sf = w2.stride()
-    grad_act = K.grouped_gemm(dy, send_token, w2, se, sf, sh, offsets, R, inter, H, pool=pool)
+    grad_act = K.grouped_gemm(dy, send_token, w2, se, sf, sh, offsets, R, inter, H, pool=pool,
+                              tiles=tiles)
     tm.end()
     # step 2: gated-activation backward
     side = _side_stream(dy.device) if overlap_act_bwd(R, offsets.numel() - 1) else None
@@ -160,7 +162,8 @@ def moe_backward_triton(saved, dy, peer_mem=None, grad_transport=None, hidden_st
     tm.end()
     # step 4: FC1 dgrad, B_e(k=j, n=h) = W1[e, h, j]; top-k reduce; gate gather
     tm.begin("fc1_dgrad")
-    dx = K.grouped_gemm(dab, None, w1, w1.stride(0), w1.stride(1), 1, offsets, R, H, 2 * inter, pool=pool)
+    dx = K.grouped_gemm(dab, None, w1, w1.stride(0), w1.stride(1), 1, offsets, R, H, 2 * inter, pool=pool,
+                        tiles=tiles)
     tm.end()
     tm.begin("combine_bwd")
     grad_hidden, grad_rw = K.combine_bwd(dx, r2s, T, k, dscale)

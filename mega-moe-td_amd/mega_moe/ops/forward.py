@@ -275,12 +275,12 @@ class FusedMoEForward(torch.nn.Module):
         self._workspaces.get(device, K.gemm_workspace_bytes(R, E), "gemm")
         self._ws_ready = True
 
-    def _route(self, selected_experts, routing_weights) -> RouteTables:
+    def _route(self, selected_experts, routing_weights, with_tiles=False) -> RouteTables:
         self._reserve_workspaces(selected_experts.device)
         num_routes = selected_experts.numel()
         need = K.route_workspace_bytes(num_routes, self.experts_per_rank)
         ws = self._workspaces.get(selected_experts.device, need, "route")
-        return route(selected_experts, self.experts_per_rank, routing_weights, ws)
+        return route(selected_experts, self.experts_per_rank, routing_weights, ws, with_tiles)
 
     # ------------------------------------------------------------ routing
     def build_routing_plan(self, selected_experts: torch.Tensor, *, moonep_plan_hook=None) -> MoERoutingPlan:
@@ -397,18 +397,18 @@ class FusedMoEForward(torch.nn.Module):
         tables = None
         if num_tokens:
             tm.begin("route")
-            tables = self._route(selected_experts, routing_weights)
+            tables = self._route(selected_experts, routing_weights, with_tiles=True)
             tm.end()
             tm.begin("fc1_swiglu")
             act, fc1_out, fc1_scale = K.fc1_swiglu(
                 hidden_states, tables.send_token, gate_up_weight, tables.offsets, tables.weight_perm, num_routes,
                 self.activation, self.situ_beta, self.situ_linear_beta, self.clamp_limit, save_fc1=return_saved,
-                fc1_dtype=self.config.save_fc1_dtype, pool=self._workspaces)
+                fc1_dtype=self.config.save_fc1_dtype, pool=self._workspaces, tiles=tables.tiles)
             tm.end()
             tm.begin("fc2")
             se, sh, sf = down_weight.stride()
             y = K.grouped_gemm(act, None, down_weight, se, sh, sf, tables.offsets, num_routes, self.hidden_size,
-                               inter, pool=self._workspaces)
+                               inter, pool=self._workspaces, tiles=tables.tiles)
             tm.end()
             tm.begin("combine")
             out = K.combine(y, tables.route_to_send, num_tokens, self.top_k)
@@ -432,7 +432,7 @@ class FusedMoEForward(torch.nn.Module):
                 expert_counts=tables.counts, split_size_cum_per_expert=tables.offsets,
                 send_route_indices=tables.send_route, send_token_indices=tables.send_token,
                 route_to_send=tables.route_to_send, recv_weights_sorted=tables.weight_perm,
-                fc1_output=fc1_out, swiglu_out_weighted=act,
+                fc1_output=fc1_out, swiglu_out_weighted=act, _tiles=tables.tiles,
             )
             if saved_recompute():
                 # MOE_SAVED_RECOMPUTE=1 (reference kernels/mega_bwd.py:3208-3226): the backward

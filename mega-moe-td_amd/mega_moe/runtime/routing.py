@@ -58,9 +58,10 @@ class RouteTables:
     """Device-resident routing tables of one pass (capacity T*k rows)."""
 
     __slots__ = ("counts", "offsets", "send_route", "send_token", "route_to_send", "weight_perm",
-                 "num_routes", "num_experts", "top_k")
+                 "tiles", "num_routes", "num_experts", "top_k")
 
-    def __init__(self, num_routes: int, num_experts: int, top_k: int, device, with_weights: bool):
+    def __init__(self, num_routes: int, num_experts: int, top_k: int, device, with_weights: bool,
+                 with_tiles: bool = False):
         i32 = dict(dtype=torch.int32, device=device)
         self.num_routes = num_routes
         self.num_experts = num_experts
@@ -72,22 +73,27 @@ class RouteTables:
         self.route_to_send = torch.empty(num_routes, **i32)
         self.weight_perm = (torch.empty(num_routes, dtype=torch.float32, device=device)
                             if with_weights else None)
+        # M-tile lists of the row GEMMs, shared by the pass's forward and backward
+        self.tiles = (torch.empty(int(_lib.load().mm_tile_lists_size(num_routes, num_experts)), dtype=torch.uint8,
+                                  device=device) if with_tiles else None)
 
 
 def route(selected_experts: torch.Tensor, num_experts: int, routing_weights: Optional[torch.Tensor],
-          workspace: torch.Tensor) -> RouteTables:
-    """Launch ``mm_route`` on the current stream; returns device tables."""
+          workspace: torch.Tensor, with_tiles: bool = False) -> RouteTables:
+    """Launch ``mm_route`` (``mm_route_tiles`` with the row GEMMs' tile lists)
+    on the current stream; returns device tables."""
     num_routes = selected_experts.numel()
     top_k = selected_experts.shape[1]
     device = selected_experts.device
-    tables = RouteTables(num_routes, num_experts, top_k, device, routing_weights is not None)
+    tables = RouteTables(num_routes, num_experts, top_k, device, routing_weights is not None, with_tiles)
     need = int(_lib.load().mm_route_workspace_bytes(num_routes, num_experts))
     if workspace.numel() < need:
         raise ValueError(f"routing workspace holds {workspace.numel()} bytes, needs {need}")
+    lists = (_lib.ptr(tables.tiles), tables.tiles.numel()) if with_tiles else ()
     _lib.call(
-        "mm_route", _lib.ptr(selected_experts), num_routes, top_k, num_experts, _lib.ptr(routing_weights),
-        _lib.ptr(tables.counts), _lib.ptr(tables.offsets), _lib.ptr(tables.send_route),
-        _lib.ptr(tables.send_token), _lib.ptr(tables.route_to_send), _lib.ptr(tables.weight_perm),
+        "mm_route_tiles" if with_tiles else "mm_route", _lib.ptr(selected_experts), num_routes, top_k, num_experts,
+        _lib.ptr(routing_weights), _lib.ptr(tables.counts), _lib.ptr(tables.offsets), _lib.ptr(tables.send_route),
+        _lib.ptr(tables.send_token), _lib.ptr(tables.route_to_send), _lib.ptr(tables.weight_perm), *lists,
         _lib.ptr(workspace), workspace.numel(), _lib.stream_of(device))
     return tables
 
