@@ -8,11 +8,12 @@
 // expert e, C_e = A_e * B_e over the rows [offsets[e], offsets[e+1]).
 //
 // MI355X design
-//  * A workgroup of 8 wavefronts (2 per SIMD; 4 for the 128 x 128 tiles)
-//    computes a BM x BN tile with v_mfma_f32_32x32x16_bf16, each wave owning
-//    a (BM / WM) x (BN / WN) sub-tile. 256 x 256 tiles with K >= 1024 run 4
-//    wavefronts of 128 x 128 (one per SIMD, accumulators in the AGPRs) with
-//    register-staged operand copies interleaved with the MFMAs.
+//  * A workgroup of 8 wavefronts (2 per SIMD) computes a BM x BN tile with
+//    v_mfma_f32_32x32x16_bf16, each wave owning a (BM / WM) x (BN / WN)
+//    sub-tile. 256 x 256 tiles with K >= 1024 run 4 wavefronts of 128 x 128
+//    (one per SIMD, accumulators in the AGPRs) with register-staged operand
+//    copies interleaved with the MFMAs. Experts averaging fewer than 96 rows
+//    run weight-streaming tiles of at most 128 rows, split by columns only.
 //  * Otherwise operands go global -> LDS with gfx950 LDS-DMA
 //    (global_load_lds_dwordx4) through an NST-stage ring, one barrier per K
 //    step. K-contiguous sources
@@ -40,6 +41,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -87,11 +89,11 @@ __device__ __forceinline__ int xcd_remap(int pid, int total) {
 
 // Grouped ordering of a (num_m x num_n) tile grid: GROUP_M M-tiles at a time
 // sweep all N tiles, so an A panel and a B tile stay hot in L2.
-__device__ __forceinline__ void grouped_mn(int l, int num_m, int num_n, int& m, int& n, int group_m = GROUP_M) {
-  const int in_group = group_m * num_n;
+__device__ __forceinline__ void grouped_mn(int l, int num_m, int num_n, int& m, int& n) {
+  const int in_group = GROUP_M * num_n;
   const int g = l / in_group;
-  const int first = g * group_m;
-  const int gs = min(num_m - first, group_m);
+  const int first = g * GROUP_M;
+  const int gs = min(num_m - first, GROUP_M);
   const int r = l - g * in_group;
   m = first + r % gs;
   n = r / gs;
@@ -179,7 +181,7 @@ struct KcTile {
   static_assert(PER_WAVE * (NT / 64) == CHUNKS, "chunks/waves mismatch");
   const bf16* ptr[PER_WAVE];
 
-  __device__ static int swz(int r) { return VPR == 8 ? ((r >> 1) & 7) : ((r >> 2) & 3); }
+  __device__ static int swz(int r) { return VPR == 16 ? (r & 15) : VPR == 8 ? ((r >> 1) & 7) : ((r >> 2) & 3); }
 
   template <class RowPtr>
   __device__ void init(RowPtr row_ptr) {
@@ -199,16 +201,9 @@ struct KcTile {
   }
   // Register-staged copy: the same vectors as issue(), loaded into VGPRs now
   // and written to the same LDS positions by put() later.
-  template <int POL = 0>
   __device__ void load(u32x4_t (&r)[PER_WAVE], int64_t k0) const {
 #pragma unroll
-    for (int v = 0; v < PER_WAVE; ++v) {
-      const u32x4_t* q = reinterpret_cast<const u32x4_t*>(ptr[v] + k0);
-      if constexpr (POL == 1)
-        r[v] = __builtin_nontemporal_load(q);
-      else
-        r[v] = *q;
-    }
+    for (int v = 0; v < PER_WAVE; ++v) r[v] = *reinterpret_cast<const u32x4_t*>(ptr[v] + k0);
   }
   __device__ static void put(bf16* lds, const u32x4_t (&r)[PER_WAVE]) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -239,8 +234,11 @@ struct MnTile {
   static constexpr int PER_WAVE = CHUNKS / (NT / 64);
   static constexpr int KPC = 64 / VPR;                      // K rows per 1 KiB chunk
   static_assert(PER_WAVE * (NT / 64) == CHUNKS, "chunks/waves mismatch");
-  static_assert(VPR >= 16, "swizzle needs >= 16 vectors per row");
+  static_assert(VPR >= 8, "swizzle needs >= 8 vectors per row");
   const bf16* ptr[PER_WAVE];
+
+  // 64-column rows: two rows per 64-bank line, so rows k and k + 2 swap halves
+  __device__ static int swz(int k) { return VPR >= 16 ? mn_swz(k) : ((k >> 1) & 1) * 4; }
 
   // K row and source column (elements) this lane copies in instruction v.
   __device__ static int k_of(int v) {
@@ -248,7 +246,7 @@ struct MnTile {
   }
   __device__ static int col_of(int v) {
     const int q = (v * (NT / 64) + (threadIdx.x >> 6)) * 64 + (threadIdx.x & 63);
-    return ((q % VPR) ^ mn_swz(q / VPR)) * 8;
+    return ((q % VPR) ^ swz(q / VPR)) * 8;
   }
   // Fixed-stride source: element (k, c) at base + k*ld + col_off(c).
   template <class ColOff>
@@ -262,16 +260,9 @@ struct MnTile {
 #pragma unroll
     for (int v = 0; v < PER_WAVE; ++v) copy16_to_lds<POL>(ptr[v] + off, lds + (v * (NT / 64) + wave) * kChunkElems);
   }
-  template <int POL = 0>
   __device__ void load(u32x4_t (&r)[PER_WAVE], int64_t off) const {
 #pragma unroll
-    for (int v = 0; v < PER_WAVE; ++v) {
-      const u32x4_t* q = reinterpret_cast<const u32x4_t*>(ptr[v] + off);
-      if constexpr (POL == 1)
-        r[v] = __builtin_nontemporal_load(q);
-      else
-        r[v] = *q;
-    }
+    for (int v = 0; v < PER_WAVE; ++v) r[v] = *reinterpret_cast<const u32x4_t*>(ptr[v] + off);
   }
   __device__ static void put(bf16* lds, const u32x4_t (&r)[PER_WAVE]) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -292,8 +283,8 @@ struct MnTile {
     const int s = lane & 15, g = lane >> 4;
     const int k = kk + 8 * (g >> 1) + (s >> 2);
     const int col = r0 + 16 * (g & 1) + 4 * (s & 3);
-    const bf16* q0 = lds + k * ROWS + ((((col >> 3) ^ mn_swz(k)) << 3) | (col & 7));
-    const bf16* q1 = lds + (k + 4) * ROWS + ((((col >> 3) ^ mn_swz(k + 4)) << 3) | (col & 7));
+    const bf16* q0 = lds + k * ROWS + ((((col >> 3) ^ swz(k)) << 3) | (col & 7));
+    const bf16* q1 = lds + (k + 4) * ROWS + ((((col >> 3) ^ swz(k + 4)) << 3) | (col & 7));
     const v4i16 lo = lds_read_tr16(q0);
     const v4i16 hi = lds_read_tr16(q1);
     const v8i16 w = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -434,8 +425,7 @@ struct RowsArgs {
   bf16* c;
   int64_t ldc;
   const TileList* tl;
-  int group_m;  // M tiles per grouped sweep of the N tiles
-  int xcd_mod;  // 1: M tile m runs on XCD m % 8 (its N tiles in order); 0: contiguous XCD shares
+  int order;  // ORDER_*
   // gated (FC1) epilogue
   const float* w;
   void* fc1_out;   // saved raw gate | up in fc1_fmt (MM_FC1_*), or null
@@ -446,19 +436,123 @@ struct RowsArgs {
   float beta, lbeta, clamp;
 };
 
+// Tile order over the workgroup ids (id b runs on XCD b % 8): contiguous
+// shares of the tile list per XCD; M tile m on XCD m % 8, its N tiles in
+// order; tile (m, n) on XCD (m * num_n + n) % 8.
+enum { ORDER_SHARES = 0, ORDER_XCD_MOD = 1, ORDER_FLAT = 2 };
 enum { EPI_STORE = 0, EPI_GATED = 1 };
 enum { B_KCONTIG = 0, B_NCONTIG = 1 };
 
-// NST-stage ring of LDS buffers: stage s is copied into buffer s % NST while
-// the MFMAs consume stage s - NST + 1; one barrier per K step.
+// Second half of the gated epilogue: the tile's bf16(gate) | bf16(up) sit in
+// LDS ([BM][BN + 8], gate in columns [0, BN / 2)); each thread turns one
+// 8-column vector of a row into act = bf16(act_fn(gate, up) * w[row]) and
+// stores it with the saved raw FC1 output.
+// w_pre(it): routing weight of row threadIdx.x / (BN / 16) + it * NT / (BN / 16).
+template <int BM, int BN, int NT, int ACT, class WFn>
+__device__ __forceinline__ void gated_store(const RowsArgs& p, const bf16* smem, int row0, int rows, int nt,
+                                            WFn w_pre) {
+  using Out = StageOut<BM, BN, NT>;
+  const int jbase = nt * (BN / 2);
+  constexpr int EPI_IT = (BM * (BN / 16) + NT - 1) / NT;
+  constexpr int VPR = BN / 16;  // 8-column vectors per output row
+  const int64_t ldf = 2 * static_cast<int64_t>(p.inter);
+  // every lane runs every pass (rows past the tile only skip their
+  // stores) so that the 16 lanes of a row can reduce the FP8 group amax
+#pragma unroll
+  for (int it = 0; it < EPI_IT; ++it) {
+    const int idx = threadIdx.x + it * NT;
+    const int r = idx / VPR, cv = idx % VPR;
+    if ((BM * VPR) % NT != 0 && r >= BM) break;  // fewer vectors than threads
+    const bool valid = r < rows;
+    const uint4 gv = *reinterpret_cast<const uint4*>(smem + r * Out::PITCH + cv * 8);
+    const uint4 uv = *reinterpret_cast<const uint4*>(smem + r * Out::PITCH + BN / 2 + cv * 8);
+    const int64_t row = row0 + r;
+    const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
+    if (valid) {
+      const float wr = w_pre(it);
+      uint32_t ow[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float a0 = gated_act(ACT, __uint_as_float(gw[q] << 16), __uint_as_float(uw[q] << 16),
+                                   p.beta, p.lbeta, p.clamp) * wr;
+        const float a1 = gated_act(ACT, __uint_as_float(gw[q] & 0xffff0000u),
+                                   __uint_as_float(uw[q] & 0xffff0000u), p.beta, p.lbeta, p.clamp) * wr;
+        ow[q] = pack_bf16x2(a0, a1);
+      }
+      store_out16(p.c + row * p.ldc + jbase + cv * 8, make_uint4(ow[0], ow[1], ow[2], ow[3]));
+    }
+    if (!p.fc1_out) continue;
+    if (p.fc1_fmt == MM_FC1_BF16) {
+      if (valid) {
+        uint16_t* fo = static_cast<uint16_t*>(p.fc1_out) + row * ldf + jbase + cv * 8;
+        store_out16(fo, gv);
+        store_out16(fo + p.inter, uv);
+      }
+    } else if (p.fc1_fmt == MM_FC1_FP16) {
+      uint32_t gh[4], uh[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        gh[q] = pack_f16x2(__uint_as_float(gw[q] << 16), __uint_as_float(gw[q] & 0xffff0000u));
+        uh[q] = pack_f16x2(__uint_as_float(uw[q] << 16), __uint_as_float(uw[q] & 0xffff0000u));
+      }
+      if (valid) {
+        uint16_t* fo = static_cast<uint16_t*>(p.fc1_out) + row * ldf + jbase + cv * 8;
+        store_out16(fo, make_uint4(gh[0], gh[1], gh[2], gh[3]));
+        store_out16(fo + p.inter, make_uint4(uh[0], uh[1], uh[2], uh[3]));
+      }
+    } else if constexpr ((BN / 2) % MM_FC1_SCALE_GROUP == 0) {
+      // FP8: one scale per row per MM_FC1_SCALE_GROUP columns of gate (and
+      // of up); a tile row holds BN / 2 of them, i.e. one or two groups.
+      // The group's 16 consecutive lanes reduce the amax of |bf16 value|
+      // with xor shuffles. (Narrower tiles never see FP8: mm_fc1_swiglu
+      // requires inter % MM_FC1_SCALE_GROUP == 0 for it, which selects
+      // 256- or 512-wide tiles.)
+      constexpr int GV = MM_FC1_SCALE_GROUP / 8;  // lanes per scale group
+      static_assert(VPR % GV == 0, "scale groups tile the row");
+      float ga = 0.0f, ua = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        ga = fmaxf(ga, fmaxf(fabsf(__uint_as_float(gw[q] << 16)), fabsf(__uint_as_float(gw[q] & 0xffff0000u))));
+        ua = fmaxf(ua, fmaxf(fabsf(__uint_as_float(uw[q] << 16)), fabsf(__uint_as_float(uw[q] & 0xffff0000u))));
+      }
+#pragma unroll
+      for (int off = 1; off < GV; off <<= 1) {
+        ga = fmaxf(ga, __shfl_xor(ga, off));
+        ua = fmaxf(ua, __shfl_xor(ua, off));
+      }
+      const float gs = ga > 0.0f ? ga : 1.0f, us = ua > 0.0f ? ua : 1.0f;
+      const float gm = kFp8Max / gs, um = kFp8Max / us;
+      uint32_t gq[2] = {0, 0}, uq[2] = {0, 0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t g0 = f32_to_e4m3fn(__uint_as_float(gw[q] << 16) * gm);
+        const uint32_t g1 = f32_to_e4m3fn(__uint_as_float(gw[q] & 0xffff0000u) * gm);
+        const uint32_t u0 = f32_to_e4m3fn(__uint_as_float(uw[q] << 16) * um);
+        const uint32_t u1 = f32_to_e4m3fn(__uint_as_float(uw[q] & 0xffff0000u) * um);
+        gq[q >> 1] |= (g0 | (g1 << 8)) << ((q & 1) * 16);
+        uq[q >> 1] |= (u0 | (u1 << 8)) << ((q & 1) * 16);
+      }
+      if (valid) {
+        uint8_t* fo = static_cast<uint8_t*>(p.fc1_out) + row * ldf + jbase + cv * 8;
+        store_out8(fo, make_uint2(gq[0], gq[1]));
+        store_out8(fo + p.inter, make_uint2(uq[0], uq[1]));
+        if (cv % GV == 0) {
+          const int groups = p.inter / MM_FC1_SCALE_GROUP;
+          float* sc = p.fc1_scale + row * (2 * groups) + (jbase + cv * 8) / MM_FC1_SCALE_GROUP;
+          sc[0] = gs / kFp8Max;
+          sc[groups] = us / kFp8Max;
+        }
+      }
+    }
+  }
+}
+
 // Epilogue of a row-GEMM tile (LDS-staged, 16-byte stores); the caller
 // has passed a barrier after the tile's last LDS reads.
-// w_pre(it): routing weight of row threadIdx.x / (BN / 16) + it * NT / (BN / 16).
 template <int BM, int BN, int NT, int EPI, int ACT, class Mma, class WFn>
 __device__ __forceinline__ void rows_epilogue(const RowsArgs& p, bf16* smem, const Mma& mma, int row0, int rows,
                                               int nt, int wm, int wn, int lane, WFn w_pre) {
   using Out = StageOut<BM, BN, NT>;
-  constexpr int EPI_VPR = BN / 16, EPI_IT = EPI == EPI_GATED ? BM * EPI_VPR / NT : 1;
   const int n0 = nt * BN;
   // The accumulators are
   // transposed (compute<..., true>): each lane stages 4 consecutive columns
@@ -476,9 +570,7 @@ __device__ __forceinline__ void rows_epilogue(const RowsArgs& p, bf16* smem, con
     Out::flush(smem, rows, p.c + static_cast<int64_t>(row0) * p.ldc + n0, p.ldc);
   } else {
     // Stage bf16(gate) in LDS columns [0, BN/2) and bf16(up) in [BN/2, BN)
-    // (tile column = output column - jbase), then each thread turns one
-    // 8-column vector of a row into act = bf16(act_fn(gate, up) * w[row]).
-    const int jbase = nt * (BN / 2);
+    // (tile column = output column - nt * BN / 2).
 #pragma unroll
     for (int i = 0; i < Mma::MI; ++i)
 #pragma unroll
@@ -490,105 +582,16 @@ __device__ __forceinline__ void rows_epilogue(const RowsArgs& p, bf16* smem, con
                     mma.acc[i][jj][4 * g], mma.acc[i][jj][4 * g + 1], mma.acc[i][jj][4 * g + 2],
                     mma.acc[i][jj][4 * g + 3]);
     __syncthreads();
-    constexpr int VPR = BN / 16;  // 8-column vectors per output row
-    const int64_t ldf = 2 * static_cast<int64_t>(p.inter);
-    // every lane runs every pass (rows past the tile only skip their
-    // stores) so that the 16 lanes of a row can reduce the FP8 group amax
-    static_assert(VPR == EPI_VPR, "epilogue vector split");
-#pragma unroll
-    for (int it = 0; it < EPI_IT; ++it) {
-      const int idx = threadIdx.x + it * NT;
-      const int r = idx / VPR, cv = idx % VPR;
-      const bool valid = r < rows;
-      const uint4 gv = *reinterpret_cast<const uint4*>(smem + r * Out::PITCH + cv * 8);
-      const uint4 uv = *reinterpret_cast<const uint4*>(smem + r * Out::PITCH + BN / 2 + cv * 8);
-      const int64_t row = row0 + r;
-      const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
-      if (valid) {
-        const float wr = w_pre(it);
-        uint32_t ow[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float a0 = gated_act(ACT, __uint_as_float(gw[q] << 16), __uint_as_float(uw[q] << 16),
-                                     p.beta, p.lbeta, p.clamp) * wr;
-          const float a1 = gated_act(ACT, __uint_as_float(gw[q] & 0xffff0000u),
-                                     __uint_as_float(uw[q] & 0xffff0000u), p.beta, p.lbeta, p.clamp) * wr;
-          ow[q] = pack_bf16x2(a0, a1);
-        }
-        store_out16(p.c + row * p.ldc + jbase + cv * 8, make_uint4(ow[0], ow[1], ow[2], ow[3]));
-      }
-      if (!p.fc1_out) continue;
-      if (p.fc1_fmt == MM_FC1_BF16) {
-        if (valid) {
-          uint16_t* fo = static_cast<uint16_t*>(p.fc1_out) + row * ldf + jbase + cv * 8;
-          store_out16(fo, gv);
-          store_out16(fo + p.inter, uv);
-        }
-      } else if (p.fc1_fmt == MM_FC1_FP16) {
-        uint32_t gh[4], uh[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          gh[q] = pack_f16x2(__uint_as_float(gw[q] << 16), __uint_as_float(gw[q] & 0xffff0000u));
-          uh[q] = pack_f16x2(__uint_as_float(uw[q] << 16), __uint_as_float(uw[q] & 0xffff0000u));
-        }
-        if (valid) {
-          uint16_t* fo = static_cast<uint16_t*>(p.fc1_out) + row * ldf + jbase + cv * 8;
-          store_out16(fo, make_uint4(gh[0], gh[1], gh[2], gh[3]));
-          store_out16(fo + p.inter, make_uint4(uh[0], uh[1], uh[2], uh[3]));
-        }
-      } else if constexpr ((BN / 2) % MM_FC1_SCALE_GROUP == 0) {
-        // FP8: one scale per row per MM_FC1_SCALE_GROUP columns of gate (and
-        // of up); a tile row holds BN / 2 of them, i.e. one or two groups.
-        // The group's 16 consecutive lanes reduce the amax of |bf16 value|
-        // with xor shuffles. (Narrower tiles never see FP8: mm_fc1_swiglu
-        // requires inter % MM_FC1_SCALE_GROUP == 0 for it, which selects
-        // 256- or 512-wide tiles.)
-        constexpr int GV = MM_FC1_SCALE_GROUP / 8;  // lanes per scale group
-        static_assert(VPR % GV == 0, "scale groups tile the row");
-        float ga = 0.0f, ua = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          ga = fmaxf(ga, fmaxf(fabsf(__uint_as_float(gw[q] << 16)), fabsf(__uint_as_float(gw[q] & 0xffff0000u))));
-          ua = fmaxf(ua, fmaxf(fabsf(__uint_as_float(uw[q] << 16)), fabsf(__uint_as_float(uw[q] & 0xffff0000u))));
-        }
-#pragma unroll
-        for (int off = 1; off < GV; off <<= 1) {
-          ga = fmaxf(ga, __shfl_xor(ga, off));
-          ua = fmaxf(ua, __shfl_xor(ua, off));
-        }
-        const float gs = ga > 0.0f ? ga : 1.0f, us = ua > 0.0f ? ua : 1.0f;
-        const float gm = kFp8Max / gs, um = kFp8Max / us;
-        uint32_t gq[2] = {0, 0}, uq[2] = {0, 0};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t g0 = f32_to_e4m3fn(__uint_as_float(gw[q] << 16) * gm);
-          const uint32_t g1 = f32_to_e4m3fn(__uint_as_float(gw[q] & 0xffff0000u) * gm);
-          const uint32_t u0 = f32_to_e4m3fn(__uint_as_float(uw[q] << 16) * um);
-          const uint32_t u1 = f32_to_e4m3fn(__uint_as_float(uw[q] & 0xffff0000u) * um);
-          gq[q >> 1] |= (g0 | (g1 << 8)) << ((q & 1) * 16);
-          uq[q >> 1] |= (u0 | (u1 << 8)) << ((q & 1) * 16);
-        }
-        if (valid) {
-          uint8_t* fo = static_cast<uint8_t*>(p.fc1_out) + row * ldf + jbase + cv * 8;
-          store_out8(fo, make_uint2(gq[0], gq[1]));
-          store_out8(fo + p.inter, make_uint2(uq[0], uq[1]));
-          if (cv % GV == 0) {
-            const int groups = p.inter / MM_FC1_SCALE_GROUP;
-            float* sc = p.fc1_scale + row * (2 * groups) + (jbase + cv * 8) / MM_FC1_SCALE_GROUP;
-            sc[0] = gs / kFp8Max;
-            sc[groups] = us / kFp8Max;
-          }
-        }
-      }
-    }
+    gated_store<BM, BN, NT, ACT>(p, smem, row0, rows, nt, w_pre);
   }
 }
 
+// NST-stage ring of LDS buffers: stage s is copied into buffer s % NST while
+// the MFMAs consume stage s - NST + 1; one barrier per K step.
 // REG: operands are loaded into VGPRs one stage ahead and written to a
 // 2-deep LDS ring with ordinary LDS stores after each stage's MFMAs (one
 // barrier per K step), instead of LDS-DMA copies.
-template <int BM, int BN, int BK_, int NST, int BLAYOUT, int EPI, int NT = kThreads, int ACT = 0, bool REG = false,
-          int BPOL = 0>
+template <int BM, int BN, int BK_, int NST, int BLAYOUT, int EPI, int NT, int ACT = 0, bool REG = false>
 __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
   constexpr int WN = 2, WM = NT / 64 / WN;  // 4 waves: 2x2, 8 waves: 4x2
   using Mma = MmaTile<BM, BN, WM, WN>;
@@ -604,16 +607,9 @@ __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
   const int num_m = p.tl->count;
   const int num_n = p.n / BN;
   int mt, nt;
-  if (p.xcd_mod) {
-    const int j = blockIdx.x / kXcds;
-    mt = (j / num_n) * kXcds + static_cast<int>(blockIdx.x % kXcds);
-    nt = j % num_n;
-    if (mt >= num_m) return;
-  } else {
-    const int l = xcd_remap(blockIdx.x, num_m * num_n);
-    if (l < 0) return;
-    grouped_mn(l, num_m, num_n, mt, nt, p.group_m);
-  }
+  const int l = xcd_remap(blockIdx.x, num_m * num_n);
+  if (l < 0) return;
+  grouped_mn(l, num_m, num_n, mt, nt);
   const int4 tile = p.tl->tiles[mt];
   const int e = tile.x, row0 = tile.y, rows = tile.z - tile.y;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -651,7 +647,7 @@ __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
   auto issue = [&](int s) {
     bf16* buf = smem + (s % NST) * STAGE;
     la.issue(buf, static_cast<int64_t>(s) * BK_);
-    lb.template issue<BPOL>(buf + ATile::ELEMS, s * b_step);
+    lb.issue(buf + ATile::ELEMS, s * b_step);
   };
 
   Mma mma;
@@ -678,7 +674,7 @@ __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
     u32x4_t ra[ATile::PER_WAVE], rb[BTile::PER_WAVE];
     auto gload = [&](int s) {
       la.load(ra, static_cast<int64_t>(s) * BK_);
-      lb.template load<BPOL>(rb, s * b_step);
+      lb.load(rb, s * b_step);
     };
     auto sput = [&](int s) {
       bf16* buf = smem + (s & 1) * STAGE;
@@ -728,7 +724,7 @@ __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
           }
           if (ss == 1) {
             BTile::put(nxt + ATile::ELEMS, rb);
-            lb.template load<BPOL>(rb, min(kt + 2, nk - 1) * b_step);
+            lb.load(rb, min(kt + 2, nk - 1) * b_step);
           }
 #pragma unroll
           for (int q = 0; q < Mma::MI * Mma::NI; ++q) {
@@ -772,6 +768,211 @@ __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
   __syncthreads();
 
   rows_epilogue<BM, BN, NT, EPI, ACT>(p, smem, mma, row0, rows, nt, wm, wn, lane, [&](int it) { return w_pre[it]; });
+}
+
+// Weight-streaming row GEMM for tiles of at most 128 rows, bound by reading
+// the weights. 8 waves split the N columns (WN of them) and, where the tile
+// has fewer than eight 32-column groups, the 16-deep K sub-steps of a stage
+// (8 / WN ways; their partial sums meet in LDS before the epilogue), so every
+// weight fragment is read from LDS once, and all waves work whatever the row
+// count. The A rows are copied and multiplied in slabs of 32, one loop per
+// slab count. Against 8 waves split 4 x 2 over 128 padded rows (us): 8
+// experts of one row, 2048 x 1536 (gate and up) 55 -> 17 and 768 x 2048 26 ->
+// 11; 117 experts of 2 rows 149 -> 116 and 69 -> 60; 256 experts' share of
+// 7168 x 4096 at 2 rows 1145 -> 976 (6.0 -> 7.0 TB/s), at 73 rows 1159 ->
+// 1081; 60 experts of 68 rows, 2304 x 1792 109 -> 92.
+template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int ACT, int WN, int BPOL>
+struct StreamRows {
+  static constexpr int NT = 512, WAVES = NT / 64, WK = WAVES / WN, NJ = BN / WN / 32, SUB = BK_ / 16;
+  static_assert(WN * WK == WAVES && NJ * WN * 32 == BN && SUB % WK == 0, "wave split");
+  using BTile = typename std::conditional<BLAYOUT == B_KCONTIG, KcTile<BN, BK_, NT>, MnTile<BN, BK_, NT>>::type;
+  static constexpr int BM = 128;
+  using Out = StageOut<BM, BN, NT>;
+  static constexpr int AVPR = BK_ / 8;  // 16-byte vectors per A row
+  static constexpr int ring(int mi) { return NST * (mi * 32 * BK_ + BTile::ELEMS); }
+  static constexpr int RED = WK > 1 ? (WK - 1) * 32 * BN * 2 : 0;  // fp32 partials of one slab, in bf16 elements
+  static constexpr int max2(int a, int b) { return a > b ? a : b; }
+  static constexpr int SMEM = max2(max2(ring(BM / 32), Out::ELEMS), RED);
+
+  // as KcTile, for any row length
+  __device__ static int a_swz(int r) { return AVPR == 4 ? ((r >> 2) & 3) : AVPR == 8 ? ((r >> 1) & 7) : (r & 15); }
+
+  template <int MI>
+  __device__ __forceinline__ static void run(const RowsArgs& p, bf16* smem, int e, int row0, int rows, int nt) {
+    constexpr int ACH = MI * 32 * BK_ / kChunkElems;     // 1 KiB chunks of A per stage
+    constexpr int PA = (ACH + WAVES - 1) / WAVES;        // per wave (a surplus wave repeats a chunk)
+    constexpr int AEL = MI * 32 * BK_;
+    constexpr int STAGE = AEL + BTile::ELEMS;
+    constexpr int LPS = PA + BTile::PER_WAVE;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wn = wave % WN, wk = wave / WN;
+    const bf16* bexp = p.b + static_cast<int64_t>(e) * p.b_se;
+    // B tile column c -> global column: gated tiles alternate 32-column groups of gate and up
+    auto bcol = [&](int c) -> int64_t {
+      if constexpr (EPI == EPI_GATED) {
+        const int g = c >> 5;
+        return static_cast<int64_t>(g & 1) * p.inter + nt * (BN / 2) + (g >> 1) * 32 + (c & 31);
+      } else {
+        return nt * BN + c;
+      }
+    };
+    BTile lb;
+    int64_t b_step;
+    if constexpr (BLAYOUT == B_KCONTIG) {
+      lb.init([&](int c) -> const bf16* { return bexp + bcol(c) * p.b_sn; });
+      b_step = BK_;
+    } else {
+      lb.init_strided(bexp, p.b_sk, bcol);
+      b_step = static_cast<int64_t>(BK_) * p.b_sk;
+    }
+    const bf16* aptr[PA];
+    int achunk[PA];
+#pragma unroll
+    for (int v = 0; v < PA; ++v) {
+      achunk[v] = (v * WAVES + wave) % ACH;
+      const int q = achunk[v] * 64 + lane, r = q / AVPR;
+      const int rr = row0 + min(r, rows - 1);  // rows past the tile re-read its last row
+      const int64_t src = p.a_rows ? static_cast<int64_t>(p.a_rows[rr]) : static_cast<int64_t>(rr);
+      aptr[v] = p.a + src * p.lda + ((q % AVPR) ^ a_swz(r)) * 8;
+    }
+    constexpr int EPI_VPR = BN / 16, EPI_IT = EPI == EPI_GATED ? (MI * 32 * EPI_VPR + NT - 1) / NT : 1;
+    float w_pre[EPI_IT];
+    if constexpr (EPI == EPI_GATED) {
+#pragma unroll
+      for (int it = 0; it < EPI_IT; ++it) {
+        const int r = (threadIdx.x + it * NT) / EPI_VPR;
+        w_pre[it] = r < rows ? p.w[row0 + r] : 0.0f;
+      }
+    }
+    auto issue = [&](int s) {
+      bf16* buf = smem + (s % NST) * STAGE;
+#pragma unroll
+      for (int v = 0; v < PA; ++v) copy16_to_lds(aptr[v] + static_cast<int64_t>(s) * BK_, buf + achunk[v] * kChunkElems);
+      lb.template issue<BPOL>(buf + AEL, s * b_step);
+    };
+    auto afrag = [&](const bf16* lds, int r0, int kk) {
+      const int r = r0 + (lane & 31), kv = (kk >> 3) + (lane >> 5);
+      return *reinterpret_cast<const bf16x8*>(lds + r * BK_ + ((kv ^ a_swz(r)) << 3));
+    };
+
+    f32x16 acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    const int nk = p.k / BK_;
+#pragma unroll
+    for (int s = 0; s < NST - 1; ++s)
+      if (s < nk) issue(s);
+    for (int kt = 0; kt < nk; ++kt) {
+      wait_stages<LPS, NST - 2>(min(nk - 1, kt + NST - 2) - kt);
+      __syncthreads();
+      if (kt + NST - 1 < nk) issue(kt + NST - 1);
+      const bf16* as = smem + (kt % NST) * STAGE;
+      const bf16* bs = as + AEL;
+#pragma unroll
+      for (int t = 0; t < SUB / WK; ++t) {
+        const int kk = (t * WK + wk) * 16;
+        bf16x8 a[MI], b[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) b[j] = BTile::frag(bs, wn * (BN / WN) + j * 32, kk, lane);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) a[i] = afrag(as, i * 32, kk);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)  // operands swapped: a lane holds 4 consecutive columns of one row
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+    if constexpr (WK > 1) {
+      float* red = reinterpret_cast<float*>(smem);  // [WK - 1][WN][NJ][16][64]
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        if (wk > 0) {
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)
+              *reinterpret_cast<f32x4*>(red + (((((wk - 1) * WN + wn) * NJ + j) * 4 + r / 4) * 64 + lane) * 4) =
+                  f32x4{acc[i][j][r], acc[i][j][r + 1], acc[i][j][r + 2], acc[i][j][r + 3]};
+        }
+        __syncthreads();
+        if (wk == 0) {
+#pragma unroll
+          for (int w = 0; w < WK - 1; ++w)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+              for (int r = 0; r < 16; r += 4) {
+                const f32x4 v =
+                    *reinterpret_cast<const f32x4*>(red + ((((w * WN + wn) * NJ + j) * 4 + r / 4) * 64 + lane) * 4);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[i][j][r + q] += v[q];
+              }
+        }
+        __syncthreads();
+      }
+    }
+    // epilogue: as rows_epilogue, with the columns split over the waves
+    using Mma = MmaTile<32, 32, 1, 1>;
+    if (wk == 0) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const int g = wn * NJ + j;  // 32-column group of the tile
+          const int c0 = EPI == EPI_GATED ? (g & 1) * (BN / 2) + (g >> 1) * 32 : g * 32;
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            Out::put4(smem, i * 32 + (lane & 31), c0 + Mma::acc_col(q, lane), acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                      acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        }
+    }
+    if constexpr (EPI == EPI_STORE) {
+      StageOut<MI * 32, BN, NT>::flush(smem, rows, p.c + static_cast<int64_t>(row0) * p.ldc + nt * BN, p.ldc);
+    } else {
+      __syncthreads();
+      gated_store<MI * 32, BN, NT, ACT>(p, smem, row0, rows, nt, [&](int it) { return w_pre[it]; });
+    }
+  }
+};
+
+template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int ACT, int WN, int BPOL>
+__global__ __launch_bounds__(512) void stream_rows_kernel(RowsArgs p) {
+  using K = StreamRows<BN, BK_, NST, BLAYOUT, EPI, ACT, WN, BPOL>;
+  __shared__ __attribute__((aligned(1024))) bf16 smem[K::SMEM];
+  const int num_n = p.n / BN;
+  const int num_m = p.tl->count;
+  int mt, nt;
+  if (p.order == ORDER_FLAT) {
+    mt = blockIdx.x / num_n;
+    nt = blockIdx.x % num_n;
+    if (mt >= num_m) return;
+  } else if (p.order == ORDER_XCD_MOD) {
+    const int j = blockIdx.x / kXcds;
+    mt = (j / num_n) * kXcds + static_cast<int>(blockIdx.x % kXcds);
+    nt = j % num_n;
+    if (mt >= num_m) return;
+  } else {
+    const int l = xcd_remap(blockIdx.x, num_m * num_n);
+    if (l < 0) return;
+    mt = l / num_n;
+    nt = l % num_n;
+  }
+  const int4 tile = p.tl->tiles[mt];
+  const int e = tile.x, row0 = tile.y, rows = tile.z - tile.y;
+  if (rows > 96)
+    K::template run<4>(p, smem, e, row0, rows, nt);
+  else if (rows > 64)
+    K::template run<3>(p, smem, e, row0, rows, nt);
+  else if (rows > 32)
+    K::template run<2>(p, smem, e, row0, rows, nt);
+  else
+    K::template run<1>(p, smem, e, row0, rows, nt);
 }
 
 // ------------------------------------------------------------------ wgrad
@@ -1361,10 +1562,23 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
 }
 
 // ------------------------------------------------------------------ host side
+// Compute units of the current device (cached per device).
+int device_cus() {
+  static int cache[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cache[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cache[dev] = n;
+  }
+  return cache[dev];
+}
+
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Row-GEMM tile choice: 256x256 when experts average at least 96 rows,
-// else a 128-row tile; 256-wide N tiles when N allows. With 129-255 rows per
+// Row-GEMM tile choice: 256x256 when experts average at least 96 rows and N
+// allows, else a weight-streaming tile of at most 128 rows. With 129-255 rows per
 // expert one 256-row tile covers an expert, so its weights stream once (two
 // 128-row tiles read them twice: Kimi-scale layer at 8192 tokens, 146 rows
 // per expert, 72.2 -> 63.0 ms per fwd+bwd step). From an average of 96 rows
@@ -1373,41 +1587,53 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 // rows per expert on average: 17.5 -> 16.4 ms per step); below that (Kimi at
 // 4096 tokens, 73 rows) it loses to the 128-row tile (43 -> 48 ms at a
 // threshold of 64).
-struct RowsCfg {
-  int bm, bn;
-};
-
-RowsCfg pick_rows_cfg(int64_t max_rows, int E, int n) {
-  RowsCfg c;
-  c.bn = (n % 256 == 0) ? 256 : 128;
-  c.bm = (c.bn == 256 && max_rows >= 96 * static_cast<int64_t>(E)) ? 256 : 128;
-  return c;
+int pick_rows_bm(int64_t max_rows, int E, int n) {
+  return n % 256 == 0 && max_rows >= 96 * static_cast<int64_t>(E) ? 256 : 128;
 }
 
-template <int BM, int BN, int BK_, int NST, int BLAYOUT, int EPI, int NT = kThreads, bool REG = false, int BPOL = 0>
+template <class Launch>
+void by_act(int kind, Launch launch) {  // activation specialised at compile time
+  if (kind == MM_ACT_SWIGLU)
+    launch(std::integral_constant<int, MM_ACT_SWIGLU>());
+  else if (kind == MM_ACT_CLAMP_SWIGLU)
+    launch(std::integral_constant<int, MM_ACT_CLAMP_SWIGLU>());
+  else
+    launch(std::integral_constant<int, MM_ACT_SITUGLU>());
+}
+
+template <int BM, int BN, int BK_, int NST, int BLAYOUT, int EPI, int NT, bool REG = false>
 void launch_rows_cfg(const RowsArgs& p, int64_t max_rows, int E, hipStream_t s) {
-  const int64_t mm = mm_max_m_tiles(max_rows, E, BM);
-  const int64_t g = p.xcd_mod ? (mm + kXcds - 1) / kXcds * kXcds * (p.n / BN) : mm * (p.n / BN);
+  const int64_t g = mm_max_m_tiles(max_rows, E, BM) * (p.n / BN);
   const int grid = static_cast<int>((g + kXcds - 1) / kXcds * kXcds);
-  if constexpr (EPI == EPI_GATED) {  // activation specialised at compile time
-    if (p.act_kind == MM_ACT_SWIGLU)
-      grouped_rows_kernel<BM, BN, BK_, NST, BLAYOUT, EPI, NT, MM_ACT_SWIGLU, REG><<<grid, NT, 0, s>>>(p);
-    else if (p.act_kind == MM_ACT_CLAMP_SWIGLU)
-      grouped_rows_kernel<BM, BN, BK_, NST, BLAYOUT, EPI, NT, MM_ACT_CLAMP_SWIGLU, REG><<<grid, NT, 0, s>>>(p);
-    else
-      grouped_rows_kernel<BM, BN, BK_, NST, BLAYOUT, EPI, NT, MM_ACT_SITUGLU, REG><<<grid, NT, 0, s>>>(p);
-  } else {
-    grouped_rows_kernel<BM, BN, BK_, NST, BLAYOUT, EPI, NT, 0, REG, BPOL><<<grid, NT, 0, s>>>(p);
-  }
+  if constexpr (EPI == EPI_GATED)
+    by_act(p.act_kind, [&](auto act) {
+      grouped_rows_kernel<BM, BN, BK_, NST, BLAYOUT, EPI, NT, decltype(act)::value, REG><<<grid, NT, 0, s>>>(p);
+    });
+  else
+    grouped_rows_kernel<BM, BN, BK_, NST, BLAYOUT, EPI, NT, 0, REG><<<grid, NT, 0, s>>>(p);
 }
 
-// 8 waves (2 per SIMD) per 128x256 workgroup by default: a second wave on
-// each SIMD keeps the matrix core busy across the other's LDS waits and
-// barriers (-7% time on the 128-row tiles of small experts against 4
-// waves). MM_GEMM_WAVES=4 selects 4 waves.
-int eight_waves() {
-  const char* e = getenv("MM_GEMM_WAVES");  // read on every call
-  return (e && strcmp(e, "4") == 0) ? 0 : 1;
+template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int WN, int BPOL>
+void launch_stream(RowsArgs p, int64_t max_rows, int E, hipStream_t s) {
+  const int64_t mm = mm_max_m_tiles(max_rows, E, 128), num_n = p.n / BN;
+  // Enough M tiles to even out over the XCDs: M tile m on XCD m % 8, its N
+  // tiles in order, so an expert's gathered A panel stays in one L2 and every
+  // XCD reads experts spread over the whole weight tensor (a contiguous
+  // eighth left some XCDs late where part of the tensor was slower to read:
+  // Kimi-scale layer -0.03 to -0.84 ms per step in five processes).
+  // MM_XCD_MOD=0 restores contiguous shares (read on every call). Few M
+  // tiles: the N tiles of each go round the XCDs.
+  p.order = mm < 64 ? ORDER_FLAT : ORDER_XCD_MOD;
+  if (const char* e = getenv("MM_XCD_MOD"))
+    if (strcmp(e, "0") == 0) p.order = ORDER_SHARES;
+  const int64_t g = p.order == ORDER_XCD_MOD ? (mm + kXcds - 1) / kXcds * kXcds * num_n : mm * num_n;
+  const int grid = static_cast<int>((g + kXcds - 1) / kXcds * kXcds);
+  if constexpr (EPI == EPI_GATED)
+    by_act(p.act_kind, [&](auto act) {
+      stream_rows_kernel<BN, BK_, NST, BLAYOUT, EPI, decltype(act)::value, WN, BPOL><<<grid, 512, 0, s>>>(p);
+    });
+  else
+    stream_rows_kernel<BN, BK_, NST, BLAYOUT, EPI, 0, WN, BPOL><<<grid, 512, 0, s>>>(p);
 }
 
 // 256x256 row tiles with K >= 1024: 4 waves of 128x128 with register-staged
@@ -1422,29 +1648,48 @@ bool rows_lds_dma() {
   return e && strcmp(e, "1") == 0;
 }
 
-// Non-temporal weight copies in the 128-row row-GEMM tiles unless
-// MM_WEIGHT_NT=0 (read on every call).
-bool weight_nt() {
+// Weight-streaming tiles (at most 128 rows of one expert): 512, 256 or 128
+// columns. A tile's time goes with its columns, times 1.15 for 256 and 1.5
+// for 128 (an expert's A rows are copied once per tile), and one workgroup
+// per CU runs them in rounds, so the width with the smallest rounds * columns
+// * factor is taken, for the experts that this many routes reach on average.
+// K-contiguous weights never take 512 (its 32-deep stages read 64-byte pieces
+// of every weight row: 3.7 against 6.5 TB/s). Measured, gate and up weights,
+// us at 512 / 256 / 128 columns: 8 experts of 2048 x 1536 45 / 24 / 17; 31:
+// 51 / 37 / 44; 56: 60 / 68 / 63; 112: 125 / 111 / 123; 14 experts of 4096 x
+// 3072 96 / 68 / 88; 32: 125 / 142 / 147.
+// The weights are read once: their copies carry the non-temporal hint, which
+// keeps them from displacing the activation rows that the expert's N tiles
+// share (112 experts of 2048 x 1536: 111 against 124 us), unless all weights
+// the call touches are small enough to be found in the 256 MiB memory-side
+// cache by the next call (8 experts, 50 MB: 17 us against 21; 16 experts, 67
+// MB: 17 against 19; 134 MB: 38 against 35).
+// MM_WEIGHT_NT=0 drops the hint (read on every call).
+struct StreamCfg {
+  int bn;
+  bool nt;
+};
+
+StreamCfg pick_stream_cfg(int64_t max_rows, int E, int n, int k, bool n_contig, bool fp8_save) {
+  const double experts = std::min({static_cast<double>(E), static_cast<double>(max_rows),
+                                   1.06 * E * (1.0 - std::exp(-static_cast<double>(max_rows) / E))});
+  const double cus = device_cus();
+  auto cost = [&](int bn, double factor) { return std::ceil(experts * (n / bn) / cus) * bn * factor; };
+  StreamCfg c{128, false};
+  double best = cost(128, 1.5);
+  if (n % 256 == 0 && (fp8_save || cost(256, 1.15) <= best)) {  // an FP8 save needs whole 128-column scale groups
+    c.bn = 256;
+    best = cost(256, 1.15);
+  }
+  if (n_contig && n % 512 == 0 && cost(512, 1.0) <= best) c.bn = 512;
   const char* e = getenv("MM_WEIGHT_NT");
-  return !(e && strcmp(e, "0") == 0);
+  c.nt = !(e && strcmp(e, "0") == 0) && experts * n * k * 2 > 96.0 * (1 << 20);
+  return c;
 }
 
 enum { WG_WIDE = 0, WG_TILE = 1, WG_LARGE = 2 };
 
 constexpr int kWideStages = 3;  // LDS: 3 x 32 KiB ring + 64 KiB staging = 160 KiB
-
-// Compute units of the current device (cached per device).
-int device_cus() {
-  static int cache[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cache[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cache[dev] = n;
-  }
-  return cache[dev];
-}
 
 // The persistent small-K weight gradient is bound by writing the gradient
 // while the K loop is short: kept up to 192 rows per expert on average
@@ -1479,7 +1724,7 @@ struct TileSource {
 template <int BLAYOUT, int EPI>
 int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const TileSource& ts, hipStream_t s,
              const char* what) {
-  const RowsCfg c = pick_rows_cfg(max_rows, E, p.n);
+  const int bm = pick_rows_bm(max_rows, E, p.n);
   // the largest grid any tile configuration launches (128-row M tiles padded
   // to a multiple of 8, 128-wide N tiles) must fit a 32-bit grid size
   if ((mm_max_m_tiles(max_rows, E, 128) + kXcds - 1) / kXcds * kXcds * (p.n / 128) >= (int64_t(1) << 31)) {
@@ -1487,65 +1732,33 @@ int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const 
     return MM_E_ARG;
   }
   if (ts.lists) {
-    p.tl = mm_tile_list_of(const_cast<void*>(ts.lists), max_rows, E, c.bm);
+    p.tl = mm_tile_list_of(const_cast<void*>(ts.lists), max_rows, E, bm);
   } else {
-    if (int rc = mm_build_tiles(offsets, E, c.bm, static_cast<TileList*>(ts.workspace), s)) return rc;
+    if (int rc = mm_build_tiles(offsets, E, bm, static_cast<TileList*>(ts.workspace), s)) return rc;
     p.tl = static_cast<const TileList*>(ts.workspace);
   }
-  // 128-row tiles (experts averaging < 256 rows, weight-streaming): one
-  // expert's N tiles run together, so its gathered A panel stays in L2
-  // (Kimi-scale: -5% layer time against 8-deep groups)
-  p.group_m = c.bm == 128 ? 1 : GROUP_M;
-  // 128-row tiles stream the weights: M tile m runs on XCD m % 8, so every
-  // XCD reads experts spread over the whole weight tensor instead of one
-  // contiguous eighth of it. Where the weights' placement made one part of
-  // the tensor slower to read, the contiguous split left some XCDs finishing
-  // late (per-workgroup clocks: XCDs 5-7 at 83-85 us per FC1-dgrad tile,
-  // 0-4 at 91-92 us); Kimi-scale layer, five processes, one-process A/B:
-  // -0.84, -0.34, -0.26, +0.03, +0.04 ms per step; alternating bench
-  // processes on a sixth box: -0.32, -0.34, -0.18 ms. MM_XCD_MOD=0 restores
-  // the contiguous split (read on every call).
-  if (c.bm == 128) {
-    const char* e = getenv("MM_XCD_MOD");
-    p.xcd_mod = !(e && strcmp(e, "0") == 0);
-  }
-  if (c.bm == 256) {
+  if (bm == 256) {
     if (rows_lds_dma() || p.k < 1024)
       launch_rows_cfg<256, 256, 64, 2, BLAYOUT, EPI, 512>(p, max_rows, E, s);
     else
       launch_rows_cfg<256, 256, 64, 2, BLAYOUT, EPI, 256, true>(p, max_rows, E, s);
-  } else if (c.bn == 256) {
-    // Weight streaming with N-contiguous weights (FC1, FC2 of small
-    // experts): 512-wide tiles halve the tile count and with it the per-tile
-    // prologue / epilogue (Kimi-scale FC1 -6%, FC2 -10%; neutral to +2% for
-    // the K-contiguous dgrads, which keep 256). BK 32 x 4 stages (4 x 40 KiB)
-    // keeps three stages of weight in flight per CU instead of one 80 KiB
-    // stage (Kimi-scale FC1 -4%, FC2 -6% against BK 64 x 2).
-    // The K-contiguous weight tiles of the 128-row dgrads are read once, so
-    // their LDS-DMA copies carry the non-temporal hint and do not displace
-    // the activation panel that every N tile of an expert reuses from L2
-    // (Kimi-scale layer, one process: FC2 dgrad 4.32 -> 4.13 ms, FC1 dgrad
-    // 9.56 -> 8.96 ms; MM_WEIGHT_NT=0 drops it). For the N-contiguous FC1 /
-    // FC2 weights it is neutral in isolation and 2.5% slower in the layer.
-    const bool wnt = BLAYOUT == B_KCONTIG && weight_nt();
-    bool wide = false;
+  } else {
+    const bool fp8_save = EPI == EPI_GATED && p.fc1_out && p.fc1_fmt == MM_FC1_FP8;
+    const StreamCfg c = pick_stream_cfg(max_rows, E, p.n, p.k, BLAYOUT == B_NCONTIG, fp8_save);
     if constexpr (BLAYOUT == B_NCONTIG) {
-      wide = p.n % 512 == 0;
-      if (wide) launch_rows_cfg<128, 512, 32, 4, BLAYOUT, EPI, 512>(p, max_rows, E, s);
-    }
-    if (!wide) {
-      // 8 waves: 32-row wave slabs, so rows past a small expert's count skip more MFMAs
-      if (eight_waves()) {
-        if (wnt)
-          launch_rows_cfg<128, 256, 64, 3, BLAYOUT, EPI, 512, false, 1>(p, max_rows, E, s);
-        else
-          launch_rows_cfg<128, 256, 64, 3, BLAYOUT, EPI, 512>(p, max_rows, E, s);
-      } else {
-        launch_rows_cfg<128, 256, 64, 3, BLAYOUT, EPI>(p, max_rows, E, s);
+      if (c.bn == 512) {
+        launch_stream<512, 32, 3, BLAYOUT, EPI, 8, 1>(p, max_rows, E, s);
+        return mm_check_launch(what);
       }
     }
-  } else {
-    launch_rows_cfg<128, 128, 64, 4, BLAYOUT, EPI>(p, max_rows, E, s);
+    if (c.bn == 256 && c.nt)
+      launch_stream<256, 64, 3, BLAYOUT, EPI, 8, 1>(p, max_rows, E, s);
+    else if (c.bn == 256)
+      launch_stream<256, 64, 3, BLAYOUT, EPI, 8, 0>(p, max_rows, E, s);
+    else if (c.nt)
+      launch_stream<128, 64, 4, BLAYOUT, EPI, 4, 1>(p, max_rows, E, s);
+    else
+      launch_stream<128, 64, 4, BLAYOUT, EPI, 4, 0>(p, max_rows, E, s);
   }
   return mm_check_launch(what);
 }
