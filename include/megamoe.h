@@ -90,7 +90,7 @@ int mm_route(const int32_t* selected, int64_t num_routes, int32_t top_k,
 
 /*
  * mm_route that also writes the M-tile lists of the row GEMMs (the expert's
- * rows cut into tiles of at most 128 and of at most 256 rows) into `tiles`
+ * rows cut into tiles of at most 160 and of at most 256 rows) into `tiles`
  * (mm_tile_lists_size(num_routes, num_experts) bytes, 16-byte aligned), so
  * that the GEMMs of the pass, forward and backward, share them
  * (mm_fc1_swiglu_tiles, mm_grouped_gemm_tiles) instead of building a list

@@ -48,15 +48,16 @@ static inline size_t mm_tile_list_bytes(int64_t max_rows, int E, int BM) {
   return mm_align_up(sizeof(TileList) + sizeof(int4) * static_cast<size_t>(mm_max_m_tiles(max_rows, E, BM)), 256);
 }
 
-// The two tile heights the row GEMMs use, in one buffer: the 128-row list,
-// then the 256-row list.
+// The two tile heights the row GEMMs use (weight-streaming and 256 x 256
+// tiles), in one buffer: the 160-row list, then the 256-row list.
+constexpr int kStreamRows = 160;
 static inline size_t mm_tile_lists_bytes(int64_t max_rows, int E) {
-  return mm_tile_list_bytes(max_rows, E, 128) + mm_tile_list_bytes(max_rows, E, 256);
+  return mm_tile_list_bytes(max_rows, E, kStreamRows) + mm_tile_list_bytes(max_rows, E, 256);
 }
 
 static inline TileList* mm_tile_list_of(void* lists, int64_t max_rows, int E, int BM) {
   char* p = static_cast<char*>(lists);
-  return reinterpret_cast<TileList*>(BM == 128 ? p : p + mm_tile_list_bytes(max_rows, E, 128));
+  return reinterpret_cast<TileList*>(BM == kStreamRows ? p : p + mm_tile_list_bytes(max_rows, E, kStreamRows));
 }
 
 // Fills one tile list from offsets (grouped_gemm.hip); the routing kernels

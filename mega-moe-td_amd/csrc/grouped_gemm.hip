@@ -12,8 +12,8 @@
 //    v_mfma_f32_32x32x16_bf16, each wave owning a (BM / WM) x (BN / WN)
 //    sub-tile. 256 x 256 tiles with K >= 1024 run 4 wavefronts of 128 x 128
 //    (one per SIMD, accumulators in the AGPRs) with register-staged operand
-//    copies interleaved with the MFMAs. Experts averaging fewer than 96 rows
-//    run weight-streaming tiles of at most 128 rows, split by columns only.
+//    copies interleaved with the MFMAs. Experts averaging fewer than 148 rows
+//    run weight-streaming tiles of at most 160 rows, split by columns only.
 //  * Otherwise operands go global -> LDS with gfx950 LDS-DMA
 //    (global_load_lds_dwordx4) through an NST-stage ring, one barrier per K
 //    step. K-contiguous sources
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
   rows_epilogue<BM, BN, NT, EPI, ACT>(p, smem, mma, row0, rows, nt, wm, wn, lane, [&](int it) { return w_pre[it]; });
 }
 
-// Weight-streaming row GEMM for tiles of at most 128 rows, bound by reading
+// Weight-streaming row GEMM for tiles of at most 160 rows, bound by reading
 // the weights. 8 waves split the N columns (WN of them) and, where the tile
 // has fewer than eight 32-column groups, the 16-deep K sub-steps of a stage
 // (8 / WN ways; their partial sums meet in LDS before the epilogue), so every
@@ -786,8 +786,9 @@ struct StreamRows {
   static constexpr int NT = 512, WAVES = NT / 64, WK = WAVES / WN, NJ = BN / WN / 32, SUB = BK_ / 16;
   static_assert(WN * WK == WAVES && NJ * WN * 32 == BN && SUB % WK == 0, "wave split");
   using BTile = typename std::conditional<BLAYOUT == B_KCONTIG, KcTile<BN, BK_, NT>, MnTile<BN, BK_, NT>>::type;
-  static constexpr int BM = 128;
-  using Out = StageOut<BM, BN, NT>;
+  static constexpr int BM = kStreamRows;
+  static constexpr int EPI_ROWS = 128;  // rows staged per epilogue pass
+  using Out = StageOut<EPI_ROWS, BN, NT>;
   static constexpr int AVPR = BK_ / 8;  // 16-byte vectors per A row
   static constexpr int ring(int mi) { return NST * (mi * 32 * BK_ + BTile::ELEMS); }
   static constexpr int RED = WK > 1 ? (WK - 1) * 32 * BN * 2 : 0;  // fp32 partials of one slab, in bf16 elements
@@ -917,26 +918,41 @@ struct StreamRows {
         __syncthreads();
       }
     }
-    // epilogue: as rows_epilogue, with the columns split over the waves
+    // epilogue: as rows_epilogue, with the columns split over the waves, in
+    // passes of at most EPI_ROWS rows
     using Mma = MmaTile<32, 32, 1, 1>;
-    if (wk == 0) {
+    constexpr int PASS = EPI_ROWS / 32;
 #pragma unroll
-      for (int i = 0; i < MI; ++i)
+    for (int i0 = 0; i0 < MI; i0 += PASS) {
+      constexpr int LAST = MI % PASS == 0 ? PASS : MI % PASS;  // slabs of the last pass
+      if (i0 > 0) __syncthreads();                             // the previous pass has left LDS
+      if (wk == 0) {
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const int g = wn * NJ + j;  // 32-column group of the tile
-          const int c0 = EPI == EPI_GATED ? (g & 1) * (BN / 2) + (g >> 1) * 32 : g * 32;
+        for (int i = i0; i < min(MI, i0 + PASS); ++i)
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            Out::put4(smem, i * 32 + (lane & 31), c0 + Mma::acc_col(q, lane), acc[i][j][4 * q], acc[i][j][4 * q + 1],
-                      acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-        }
-    }
-    if constexpr (EPI == EPI_STORE) {
-      StageOut<MI * 32, BN, NT>::flush(smem, rows, p.c + static_cast<int64_t>(row0) * p.ldc + nt * BN, p.ldc);
-    } else {
-      __syncthreads();
-      gated_store<MI * 32, BN, NT, ACT>(p, smem, row0, rows, nt, [&](int it) { return w_pre[it]; });
+          for (int j = 0; j < NJ; ++j) {
+            const int g = wn * NJ + j;  // 32-column group of the tile
+            const int c0 = EPI == EPI_GATED ? (g & 1) * (BN / 2) + (g >> 1) * 32 : g * 32;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              Out::put4(smem, (i - i0) * 32 + (lane & 31), c0 + Mma::acc_col(q, lane), acc[i][j][4 * q],
+                        acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+          }
+      }
+      const int r0 = row0 + i0 * 32, nr = rows - i0 * 32;
+      auto w_of = [&](int it) { return w_pre[i0 * 32 * EPI_VPR / NT + it]; };
+      if constexpr (EPI == EPI_STORE) {
+        if (i0 + PASS < MI)
+          Out::flush(smem, min(nr, EPI_ROWS), p.c + static_cast<int64_t>(r0) * p.ldc + nt * BN, p.ldc);
+        else
+          StageOut<LAST * 32, BN, NT>::flush(smem, nr, p.c + static_cast<int64_t>(r0) * p.ldc + nt * BN, p.ldc);
+      } else {
+        __syncthreads();
+        if (i0 + PASS < MI)
+          gated_store<EPI_ROWS, BN, NT, ACT>(p, smem, r0, min(nr, EPI_ROWS), nt, w_of);
+        else
+          gated_store<LAST * 32, BN, NT, ACT>(p, smem, r0, nr, nt, w_of);
+      }
     }
   }
 };
@@ -965,7 +981,9 @@ __global__ __launch_bounds__(512) void stream_rows_kernel(RowsArgs p) {
   }
   const int4 tile = p.tl->tiles[mt];
   const int e = tile.x, row0 = tile.y, rows = tile.z - tile.y;
-  if (rows > 96)
+  if (rows > 128)
+    K::template run<5>(p, smem, e, row0, rows, nt);
+  else if (rows > 96)
     K::template run<4>(p, smem, e, row0, rows, nt);
   else if (rows > 64)
     K::template run<3>(p, smem, e, row0, rows, nt);
@@ -1577,18 +1595,17 @@ int device_cus() {
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Row-GEMM tile choice: 256x256 when experts average at least 96 rows and N
-// allows, else a weight-streaming tile of at most 128 rows. With 129-255 rows per
-// expert one 256-row tile covers an expert, so its weights stream once (two
-// 128-row tiles read them twice: Kimi-scale layer at 8192 tokens, 146 rows
-// per expert, 72.2 -> 63.0 ms per fwd+bwd step). From an average of 96 rows
-// per expert on, softmax top-k routing puts about half the experts above 128
-// rows, so the 256-row tile already pays (E=256 top-8 at 4096 tokens, 128
-// rows per expert on average: 17.5 -> 16.4 ms per step); below that (Kimi at
-// 4096 tokens, 73 rows) it loses to the 128-row tile (43 -> 48 ms at a
-// threshold of 64).
+// Row-GEMM tile height: weight-streaming tiles of at most 160 rows while
+// experts average fewer than 148 rows (or N is no multiple of 256), 256 x 256
+// tiles above. Either way an expert's weights should be read once, so the
+// streaming tile must hold most experts: 160 rows hold an average of 128 with
+// softmax top-k routing, and past 148 half the experts would need a second
+// tile. Measured, us streaming / 256 x 256, 128 experts: FC1 of 7168 x 4096
+// at 96 rows 1195 / 1419, 128 rows 1363 / 1580, 146 rows 1554 / 1699; FC2 of
+// 2048 x 7168 624 / 784, 700 / 882, 791 / 932; 2048 x 1536 at 140 rows 192 /
+// 201, 150 rows 212 / 208, 170 rows 284 / 207.
 int pick_rows_bm(int64_t max_rows, int E, int n) {
-  return n % 256 == 0 && max_rows >= 96 * static_cast<int64_t>(E) ? 256 : 128;
+  return n % 256 == 0 && max_rows >= 148 * static_cast<int64_t>(E) ? 256 : kStreamRows;
 }
 
 template <class Launch>
@@ -1615,7 +1632,7 @@ void launch_rows_cfg(const RowsArgs& p, int64_t max_rows, int E, hipStream_t s) 
 
 template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int WN, int BPOL>
 void launch_stream(RowsArgs p, int64_t max_rows, int E, hipStream_t s) {
-  const int64_t mm = mm_max_m_tiles(max_rows, E, 128), num_n = p.n / BN;
+  const int64_t mm = mm_max_m_tiles(max_rows, E, kStreamRows), num_n = p.n / BN;
   // Enough M tiles to even out over the XCDs: M tile m on XCD m % 8, its N
   // tiles in order, so an expert's gathered A panel stays in one L2 and every
   // XCD reads experts spread over the whole weight tensor (a contiguous
@@ -1648,7 +1665,7 @@ bool rows_lds_dma() {
   return e && strcmp(e, "1") == 0;
 }
 
-// Weight-streaming tiles (at most 128 rows of one expert): 512, 256 or 128
+// Weight-streaming tiles (at most 160 rows of one expert): 512, 256 or 128
 // columns. A tile's time goes with its columns, times 1.15 for 256 and 1.5
 // for 128 (an expert's A rows are copied once per tile), and one workgroup
 // per CU runs them in rounds, so the width with the smallest rounds * columns
@@ -1670,14 +1687,17 @@ struct StreamCfg {
   bool nt;
 };
 
-StreamCfg pick_stream_cfg(int64_t max_rows, int E, int n, int k, bool n_contig, bool fp8_save) {
+StreamCfg pick_stream_cfg(int64_t max_rows, int E, int n, int k, bool n_contig, bool save) {
   const double experts = std::min({static_cast<double>(E), static_cast<double>(max_rows),
                                    1.06 * E * (1.0 - std::exp(-static_cast<double>(max_rows) / E))});
   const double cus = device_cus();
   auto cost = [&](int bn, double factor) { return std::ceil(experts * (n / bn) / cus) * bn * factor; };
   StreamCfg c{128, false};
   double best = cost(128, 1.5);
-  if (n % 256 == 0 && (fp8_save || cost(256, 1.15) <= best)) {  // an FP8 save needs whole 128-column scale groups
+  // a call that saves FC1 takes at least 256 columns: an FP8 save needs whole
+  // 128-column scale groups, and every format then narrows the same fp32 sums
+  // (128 columns split K over two waves, which sums in another order)
+  if (n % 256 == 0 && (save || cost(256, 1.15) <= best)) {
     c.bn = 256;
     best = cost(256, 1.15);
   }
@@ -1725,9 +1745,9 @@ template <int BLAYOUT, int EPI>
 int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const TileSource& ts, hipStream_t s,
              const char* what) {
   const int bm = pick_rows_bm(max_rows, E, p.n);
-  // the largest grid any tile configuration launches (128-row M tiles padded
-  // to a multiple of 8, 128-wide N tiles) must fit a 32-bit grid size
-  if ((mm_max_m_tiles(max_rows, E, 128) + kXcds - 1) / kXcds * kXcds * (p.n / 128) >= (int64_t(1) << 31)) {
+  // the largest grid any tile configuration launches (the shortest M tiles
+  // padded to a multiple of 8, 128-wide N tiles) must fit a 32-bit grid size
+  if ((mm_max_m_tiles(max_rows, E, kStreamRows) + kXcds - 1) / kXcds * kXcds * (p.n / 128) >= (int64_t(1) << 31)) {
     mm_set_error("%s: too many tiles for one launch", what);
     return MM_E_ARG;
   }
@@ -1743,8 +1763,7 @@ int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const 
     else
       launch_rows_cfg<256, 256, 64, 2, BLAYOUT, EPI, 256, true>(p, max_rows, E, s);
   } else {
-    const bool fp8_save = EPI == EPI_GATED && p.fc1_out && p.fc1_fmt == MM_FC1_FP8;
-    const StreamCfg c = pick_stream_cfg(max_rows, E, p.n, p.k, BLAYOUT == B_NCONTIG, fp8_save);
+    const StreamCfg c = pick_stream_cfg(max_rows, E, p.n, p.k, BLAYOUT == B_NCONTIG, p.fc1_out != nullptr);
     if constexpr (BLAYOUT == B_NCONTIG) {
       if (c.bn == 512) {
         launch_stream<512, 32, 3, BLAYOUT, EPI, 8, 1>(p, max_rows, E, s);
@@ -1773,7 +1792,7 @@ int mm_build_tiles(const int32_t* offsets, int E, int BM, TileList* tl, hipStrea
 namespace {
 
 int check_tile_source(const TileSource& ts, int64_t max_rows, int E, const char* what) {
-  const size_t need = ts.lists ? mm_tile_lists_bytes(max_rows, E) : mm_tile_list_bytes(max_rows, E, 128);
+  const size_t need = ts.lists ? mm_tile_lists_bytes(max_rows, E) : mm_tile_list_bytes(max_rows, E, kStreamRows);
   if ((!ts.lists && !ts.workspace) || ts.bytes < need) {
     mm_set_error("%s: %s too small", what, ts.lists ? "tile lists" : "workspace");
     return MM_E_WS;
@@ -1896,7 +1915,7 @@ extern "C" int mm_grouped_gemm_tiles(const uint16_t* a, int64_t lda, const int32
 }
 
 extern "C" size_t mm_gemm_workspace_bytes(int64_t max_rows, int32_t num_experts) {
-  return mm_tile_list_bytes(max_rows, num_experts, 128);  // 128 rows: the longer of the two lists
+  return mm_tile_list_bytes(max_rows, num_experts, kStreamRows);  // the longer of the two lists
 }
 
 // Every weight-gradient kernel gathers its rows in place: no workspace.

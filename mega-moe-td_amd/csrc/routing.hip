@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
     const int32_t* __restrict__ sel, int64_t R, int top_k, int E, int nbits, int nunits,
     const int32_t* __restrict__ unit_counts, const float* __restrict__ rw, int32_t* __restrict__ counts,
     int32_t* __restrict__ offsets, int32_t* __restrict__ send_route, int32_t* __restrict__ send_token,
-    int32_t* __restrict__ route_to_send, float* __restrict__ weight_perm, TileList* __restrict__ tl128,
+    int32_t* __restrict__ route_to_send, float* __restrict__ weight_perm, TileList* __restrict__ tlS,
     TileList* __restrict__ tl256) {
   __shared__ int seg[kFusedWaves * kFusedExperts];  // [wave][expert]: routes of the segment, then its next row
   __shared__ int before[kFusedExperts], rest[kFusedExperts];  // routes in earlier / later units
@@ -217,17 +217,18 @@ __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
       if (tid == E - 1) offsets[E] = first + total;
     }
   }
-  if (u == nunits - 1 && tl128) {
-    const uint64_t t128 = (total + 127) / 128, t256 = (total + 255) / 256;
-    const uint64_t t = block_scan(t128 | (t256 << 32), part);
+  if (u == nunits - 1 && tlS) {
+    const uint64_t tS = (total + kStreamRows - 1) / kStreamRows, t256 = (total + 255) / 256;
+    const uint64_t t = block_scan(tS | (t256 << 32), part);
     if (tid < E) {
-      int n = static_cast<int>(t & 0xffffffffu) - static_cast<int>(t128);
-      for (int r = 0; r < total; r += 128) tl128->tiles[n++] = make_int4(tid, first + r, first + min(r + 128, total), 0);
+      int n = static_cast<int>(t & 0xffffffffu) - static_cast<int>(tS);
+      for (int r = 0; r < total; r += kStreamRows)
+        tlS->tiles[n++] = make_int4(tid, first + r, first + min(r + kStreamRows, total), 0);
       n = static_cast<int>(t >> 32) - static_cast<int>(t256);
       for (int r = 0; r < total; r += 256) tl256->tiles[n++] = make_int4(tid, first + r, first + min(r + 256, total), 0);
     }
     if (tid == kFusedThreads - 1) {
-      tl128->count = static_cast<int>(t & 0xffffffffu);
+      tlS->count = static_cast<int>(t & 0xffffffffu);
       tl256->count = static_cast<int>(t >> 32);
     }
   }
@@ -332,7 +333,7 @@ int route_launch(const int32_t* selected, int64_t num_routes, int32_t top_k, int
   const int E = num_experts;
   const int nunits = static_cast<int>((num_routes + kChunk - 1) / kChunk);
   const int nbits = 32 - __builtin_clz(static_cast<unsigned>(E));
-  TileList* tl128 = tiles ? mm_tile_list_of(tiles, num_routes, E, 128) : nullptr;
+  TileList* tlS = tiles ? mm_tile_list_of(tiles, num_routes, E, kStreamRows) : nullptr;
   TileList* tl256 = tiles ? mm_tile_list_of(tiles, num_routes, E, 256) : nullptr;
   if (E <= kFusedExperts) {
     const bool recount = recount_routes(num_routes, E);
@@ -340,7 +341,7 @@ int route_launch(const int32_t* selected, int64_t num_routes, int32_t top_k, int
       route_count_kernel<<<nunits, kThreads, E * sizeof(int), s>>>(selected, num_routes, E, nunits, unit_counts);
     route_fused_kernel<<<nunits > 0 ? nunits : 1, kFusedThreads, 0, s>>>(
         selected, num_routes, top_k, E, nbits, nunits > 0 ? nunits : 1, recount ? nullptr : unit_counts,
-        routing_weights, counts, offsets, send_route, send_token, route_to_send, weight_perm, tl128, tl256);
+        routing_weights, counts, offsets, send_route, send_token, route_to_send, weight_perm, tlS, tl256);
     return mm_check_launch(what);
   }
   // dynamic LDS above 64 KiB (up to 132 KiB at kMaxExperts); set once
@@ -363,7 +364,7 @@ int route_launch(const int32_t* selected, int64_t num_routes, int32_t top_k, int
         route_to_send, weight_perm);
   if (int rc = mm_check_launch(what)) return rc;
   if (tiles) {
-    if (int rc = mm_build_tiles(offsets, E, 128, tl128, s)) return rc;
+    if (int rc = mm_build_tiles(offsets, E, kStreamRows, tlS, s)) return rc;
     return mm_build_tiles(offsets, E, 256, tl256, s);
   }
   return MM_OK;

@@ -30,7 +30,7 @@ CASES = [
 def _lists(buf, max_rows, E, offsets):
     """(device list, expected list) of both tile heights."""
     off = 0
-    for bm in (128, 256):
+    for bm in (160, 256):
         cap = max_rows // bm + min(E, max_rows)
         words = buf[off:off + 16 + 16 * cap].view(torch.int32).cpu().numpy()
         n = int(words[0])
