@@ -299,6 +299,64 @@ int mm_gated_act(const void* fc1_out, int64_t ld_fc1, int32_t fc1_format,
                  float situ_linear_beta, float clamp_limit, uint16_t* act,
                  int64_t ld_act, mm_stream_t stream);
 
+/* ---------------------------------------------------------- whole layer */
+
+/*
+ * The forward of the layer in one call: mm_route_tiles, mm_fc1_swiglu_tiles,
+ * mm_grouped_gemm_tiles (FC2) and mm_combine on one stream, bit-identical to
+ * calling them in turn. x [tokens, hidden], selected / routing_weights
+ * [tokens, top_k], w1 [E, H, 2I], all contiguous; w2 element (e, h, f) at
+ * e*w2_se + h*w2_sh + f*w2_sf; out [tokens, hidden]. With counts != NULL
+ * (all tables, tiles of mm_tile_lists_size(tokens * top_k, E) bytes, and act
+ * given; fc1_out and fc1_scale as in mm_fc1_swiglu) the pass's tables and
+ * activations are the caller's to keep for mm_moe_backward; with all of them
+ * NULL they live in scratch (mm_moe_forward_scratch_bytes with keep_tables =
+ * counts != NULL; 0 for sizes out of range), which is free again when the
+ * stream has passed the call. Replaces the launches of ops/forward.py:
+ * 1884-2109.
+ */
+size_t mm_moe_forward_scratch_bytes(int64_t tokens, int32_t top_k,
+                                    int32_t num_experts, int32_t hidden,
+                                    int32_t inter, int32_t keep_tables);
+
+int mm_moe_forward(const uint16_t* x, const int32_t* selected,
+                   const float* routing_weights, const uint16_t* w1,
+                   const uint16_t* w2, int64_t w2_se, int64_t w2_sh, int64_t w2_sf,
+                   int64_t tokens, int32_t top_k, int32_t num_experts,
+                   int32_t hidden, int32_t inter, int32_t act_kind,
+                   float situ_beta, float situ_linear_beta, float clamp_limit,
+                   int32_t* counts, int32_t* offsets, int32_t* send_route,
+                   int32_t* send_token, int32_t* route_to_send,
+                   float* weight_perm, void* tiles, size_t tiles_bytes,
+                   uint16_t* act, void* fc1_out, int32_t fc1_format,
+                   float* fc1_scale, uint16_t* out, void* scratch,
+                   size_t scratch_bytes, mm_stream_t stream);
+
+/*
+ * The five backward stages in one call on one stream, from what
+ * mm_moe_forward kept: FC2 dgrad (grad_act [R, I]), gated-activation backward
+ * (dab [R, 2I], dscale [R]), with recompute_act != 0 the activation recompute
+ * into act (read otherwise), FC2 wgrad (grad_fc2 [E, H, I]), FC1 dgrad (dx
+ * [R, H]), top-k reduce and routing-weight gradient (grad_hidden [T, H],
+ * grad_rw [T, k]), FC1 wgrad (grad_gate_up [E, H, 2I]). All row-major
+ * contiguous, R = tokens * top_k. Replaces the launches of
+ * ops/backward.py:100-399.
+ */
+int mm_moe_backward(const uint16_t* dy, const uint16_t* x, const uint16_t* w1,
+                    const uint16_t* w2, int64_t w2_se, int64_t w2_sh,
+                    int64_t w2_sf, int64_t tokens, int32_t top_k,
+                    int32_t num_experts, int32_t hidden, int32_t inter,
+                    int32_t act_kind, float situ_beta, float situ_linear_beta,
+                    float clamp_limit, const int32_t* offsets,
+                    const int32_t* send_token, const int32_t* route_to_send,
+                    const float* weight_perm, const void* tiles,
+                    size_t tiles_bytes, const void* fc1_out,
+                    int32_t fc1_format, const float* fc1_scale, uint16_t* act,
+                    int32_t recompute_act, uint16_t* grad_act, uint16_t* dab,
+                    uint16_t* dscale, uint16_t* grad_fc2, uint16_t* dx,
+                    uint16_t* grad_hidden, float* grad_rw,
+                    uint16_t* grad_gate_up, mm_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -55,6 +55,13 @@ SIGNATURES = {
     "mm_combine_bwd": (ctypes.c_int, [_P, _I64, _P, _I64, _I32, _I32, _P, _I64, _P, _P, _P]),
     "mm_gated_act": (ctypes.c_int, [_P, _I64, _I32, _P, _P, _P, _I32, _I64, _I32, _I32, _F32, _F32, _F32, _P,
                                     _I64, _P]),
+    "mm_moe_forward_scratch_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32, _I32]),
+    "mm_moe_forward": (ctypes.c_int, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32,
+                                      _F32, _F32, _F32, _P, _P, _P, _P, _P, _P, _P, _SZ, _P, _P, _I32, _P, _P, _P,
+                                      _SZ, _P]),
+    "mm_moe_backward": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _F32,
+                                       _F32, _F32, _P, _P, _P, _P, _P, _SZ, _P, _I32, _P, _P, _I32, _P, _P, _P, _P,
+                                       _P, _P, _P, _P, _P]),
     "mm_swiglu_bwd": (ctypes.c_int, [_P, _I64, _P, _I64, _I32, _P, _P, _P, _I32, _I64, _I32, _I32, _F32,
                                      _F32, _F32, _P, _P, _P]),
 }

@@ -260,3 +260,69 @@ def gated_act(fc1_out, weight_perm, offsets, max_rows: int, activation: str, sit
               offsets.numel() - 1, max_rows, inter, _lib.ACT_KINDS[activation], float(situ_beta), lbeta,
               float(clamp_limit), _lib.ptr(act), act.stride(0), _lib.stream_of(fc1_out.device))
     return act
+
+
+def layer_forward(x, selected, routing_weights, w1, w2, num_experts: int, activation: str, situ_beta: float,
+                  situ_linear_beta, clamp_limit: float, tables, fc1_dtype: str, stream: int):
+    """Routing, FC1 + gated activation, FC2 and combine in one call on ``stream``
+    (``mm_moe_forward``), for operands the operator has validated.
+
+    ``tables`` (``RouteTables`` with weights and tile lists) receives the
+    routing tables of a pass whose activations are kept; with ``None`` they
+    live in the call's scratch. Returns (out, act, fc1_output, fc1_scale), the
+    last three ``None`` without ``tables``.
+    """
+    tokens, top_k = selected.shape
+    hidden, inter = x.shape[1], w1.shape[2] // 2
+    dev, lib = x.device, _lib.load()
+    out = torch.empty(tokens, hidden, dtype=torch.bfloat16, device=dev)
+    act = fc1_out = fc1_scale = None
+    fmt = 0
+    if tables is None:
+        kept = (None, None, None, None, None, None, None, 0, None, None)
+    else:
+        rows = tokens * top_k
+        act = torch.empty(rows, inter, dtype=torch.bfloat16, device=dev)
+        fc1_out = torch.empty(rows, 2 * inter, dtype=_FC1_TORCH_DTYPE[fc1_dtype], device=dev)
+        fmt = _lib.FC1_FORMATS[fc1_dtype]
+        if fc1_dtype == "fp8":
+            fc1_scale = torch.empty(rows, 2 * inter // _lib.FC1_SCALE_GROUP, dtype=torch.float32, device=dev)
+        kept = (tables.counts.data_ptr(), tables.offsets.data_ptr(), tables.send_route.data_ptr(),
+                tables.send_token.data_ptr(), tables.route_to_send.data_ptr(), tables.weight_perm.data_ptr(),
+                tables.tiles.data_ptr(), tables.tiles.numel(), act.data_ptr(), fc1_out.data_ptr())
+    nbytes = lib.mm_moe_forward_scratch_bytes(tokens, top_k, num_experts, hidden, inter, tables is not None)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    se, sh, sf = w2.stride()
+    _lib.call("mm_moe_forward", x.data_ptr(), selected.data_ptr(), routing_weights.data_ptr(), w1.data_ptr(),
+              w2.data_ptr(), se, sh, sf, tokens, top_k, num_experts, hidden, inter, _lib.ACT_KINDS[activation],
+              situ_beta, situ_linear_beta if situ_linear_beta is not None else 0.0, clamp_limit, *kept, fmt,
+              None if fc1_scale is None else fc1_scale.data_ptr(), out.data_ptr(), scratch.data_ptr(), nbytes, stream)
+    return out, act, fc1_out, fc1_scale
+
+
+def layer_backward(dy, x, w1, w2, tokens: int, top_k: int, offsets, send_token, route_to_send, weight_perm, tiles,
+                   fc1_out, fc1_scale, act, activation: str, situ_beta: float, situ_linear_beta, clamp_limit: float):
+    """The five backward stages in one call on the current stream
+    (``mm_moe_backward``); ``act`` is recomputed from ``fc1_out`` when ``None``.
+    Returns (grad_act, dab, dscale, grad_fc2, dx, grad_hidden, grad_rw, grad_gate_up).
+    """
+    num_experts, hidden, two_inter = w1.shape
+    inter, rows = two_inter // 2, tokens * top_k
+    bf = dict(dtype=torch.bfloat16, device=dy.device)
+    recompute = act is None
+    if recompute:
+        act = torch.empty(rows, inter, **bf)
+    grad_act, dab, dscale = torch.empty(rows, inter, **bf), torch.empty(rows, two_inter, **bf), torch.empty(rows, **bf)
+    grad_fc2, dx = torch.empty(num_experts, hidden, inter, **bf), torch.empty(rows, hidden, **bf)
+    gh, ggu = torch.empty(tokens, hidden, **bf), torch.empty(num_experts, hidden, two_inter, **bf)
+    grw = torch.empty(tokens, top_k, dtype=torch.float32, device=dy.device)
+    se, sh, sf = w2.stride()
+    _lib.call("mm_moe_backward", dy.data_ptr(), x.data_ptr(), w1.data_ptr(), w2.data_ptr(), se, sh, sf, tokens, top_k,
+              num_experts, hidden, inter, _lib.ACT_KINDS[activation], situ_beta,
+              situ_linear_beta if situ_linear_beta is not None else 0.0, clamp_limit, offsets.data_ptr(),
+              send_token.data_ptr(), route_to_send.data_ptr(), weight_perm.data_ptr(), tiles.data_ptr(),
+              tiles.numel(), fc1_out.data_ptr(), _lib.FC1_FORMATS[fc1_format_of(fc1_out)],
+              None if fc1_scale is None else fc1_scale.data_ptr(), act.data_ptr(), recompute, grad_act.data_ptr(),
+              dab.data_ptr(), dscale.data_ptr(), grad_fc2.data_ptr(), dx.data_ptr(), gh.data_ptr(), grw.data_ptr(),
+              ggu.data_ptr(), torch.cuda.current_stream(dy.device).cuda_stream)
+    return grad_act, dab, dscale, grad_fc2, dx, gh, grw, ggu

@@ -64,6 +64,34 @@ def _side_stream(device) -> torch.cuda.Stream:
     return st
 
 
+def _one_call(saved, dy, x, tiles) -> bool:
+    """Whether the pass can go through ``mm_moe_backward``: the saved tensors
+    as the forward wrote them, on one device. Anything else takes the staged
+    calls, which check (and refuse) operand by operand."""
+    R, F, dev = saved["total_routes"], saved["ffn_dim"], dy.device
+    E, H = saved["gate_up_weight"].shape[0], saved["hidden_dim"]
+    i32, bf = torch.int32, torch.bfloat16
+    fc1, act = saved["fc1_output"], dict.get(saved, "swiglu_out_weighted")
+
+    def plain(t, dtype, shape):
+        return t is not None and t.dtype == dtype and t.device == dev and t.shape == shape and t.is_contiguous()
+
+    if tiles is None or dev.type != "cuda" or fc1.dtype not in (bf, torch.float16, torch.float8_e4m3fn):
+        return False
+    if fc1.dtype == torch.float8_e4m3fn and not (
+            int(saved.get("fc1_scale_group_size", 0)) == 128
+            and plain(saved.get("fc1_output_scale"), torch.float32, (R, 2 * F // 128))):
+        return False
+    w2 = saved["down_weight"]
+    return (x.device == dev and tiles.device == dev and plain(fc1, fc1.dtype, (R, 2 * F))
+            and plain(saved["gate_up_weight"], bf, (E, H, 2 * F))
+            and w2.dtype == bf and w2.device == dev and w2.shape == (E, H, F)
+            and (act is None or plain(act, bf, (R, F)))
+            and plain(saved["recv_weights_sorted"], torch.float32, (R,))
+            and plain(saved["split_size_cum_per_expert"], i32, (E + 1,))
+            and plain(saved["send_token_indices"], i32, (R,)) and plain(saved["route_to_send"], i32, (R,)))
+
+
 def moe_backward_triton(saved, dy, peer_mem=None, grad_transport=None, hidden_states=None):
     """Run the five backward stages on a ``saved`` dict from ``FusedMoEForward``.
 
@@ -106,6 +134,15 @@ def moe_backward_triton(saved, dy, peer_mem=None, grad_transport=None, hidden_st
     pool = saved.get("_workspaces")
     ws_rows = saved.get("_max_routes") or R
     tiles = saved.get("_tiles")
+    side = _side_stream(dy.device) if overlap_act_bwd(R, offsets.numel() - 1) else None
+    if side is None and tm is NULL_TIMER and _one_call(saved, dy, x, tiles):
+        act = None if saved_recompute() else saved.get("swiglu_out_weighted")
+        grad_act, dab, dscale, grad_fc2, dx, grad_hidden, grad_rw, grad_gate_up = K.layer_backward(
+            dy, x, w1, w2, T, k, offsets, send_token, r2s, saved["recv_weights_sorted"], tiles, saved["fc1_output"],
+            saved.get("fc1_output_scale"), act, **act_kw)
+        grads = _grad_dict(grad_hidden, grad_rw, grad_fc2, grad_gate_up, grad_act, dab, dscale, inter)
+        grads._bind(dy, send_token, offsets, dx if saved.get("_keep_grad_recv_hidden_sorted") else None)
+        return grads
     # step 1: FC2 dgrad, B_e(k=h, n=f) = down[e, h, f]
     tm.begin("fc2_dgrad")
     se, sh, sf = w2.stride()
@@ -113,7 +150,6 @@ def moe_backward_triton(saved, dy, peer_mem=None, grad_transport=None, hidden_st
                               tiles=tiles)
     tm.end()
     # step 2: gated-activation backward
-    side = _side_stream(dy.device) if overlap_act_bwd(R, offsets.numel() - 1) else None
     if side is None:  # overlapped with step 3 otherwise: its time is part of "fc2_wgrad"
         tm.begin("swiglu_bwd")
     fc1_scale = None

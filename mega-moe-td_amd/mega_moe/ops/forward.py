@@ -5,9 +5,10 @@ Public surface and validation follow the reference operator
 :853-884, ``dispatch_fc1`` :928-1320, ``forward`` :1884-2109, validators
 :766-850, ``pack_gate_up_weights`` :2112-2137, ``DispatchFC1Result`` :57-65.
 
-Pipeline of ``forward`` (all on the caller's stream, no host sync):
+Pipeline of ``forward`` (all on the caller's stream, no host sync; one call,
+``mm_moe_forward``, issues the four launches unless a stage timer is attached):
 
-    mm_route       selected_experts -> expert-major tables + permuted weights
+    mm_route_tiles selected_experts -> expert-major tables, permuted weights, tile lists
     mm_fc1_swiglu  rows gathered from hidden_states by send_token (the
                    one-GPU dispatch is fused into the A-tile load) @ W1[e],
                    weighted gated activation in the epilogue -> act [R, I]
@@ -31,7 +32,7 @@ import torch.distributed
 from ..config import MoEForwardConfig
 from ..runtime.routing import MoERoutingPlan, RouteTables, plan_from_tables, route
 from ._saved import MoESaved
-from ..runtime.timing import NULL_TIMER, StageTimer
+from ..runtime.timing import StageTimer
 from . import _kernels as K
 
 # Device-kernel limits (csrc/routing.hip kMaxExperts, csrc/rowops.hip combine slots).
@@ -231,6 +232,7 @@ class FusedMoEForward(torch.nn.Module):
         elif self._forward_stream != current:
             raise RuntimeError(
                 "FusedMoEForward is single-stream; recreate the operator for a different caller stream")
+        return current
 
     # ------------------------------------------------------------ lifecycle
     def sync(self):
@@ -368,6 +370,33 @@ class FusedMoEForward(torch.nn.Module):
         )
 
     # ------------------------------------------------------------ full forward
+    def _forward_staged(self, hidden_states, selected_experts, gate_up_weight, down_weight, routing_weights,
+                        return_saved):
+        """The launches of ``mm_moe_forward`` one entry point at a time, with
+        the stage timer's events between them."""
+        tm = self.stage_timer
+        num_tokens = hidden_states.shape[0]
+        num_routes = num_tokens * self.top_k
+        inter = gate_up_weight.shape[2] // 2
+        tm.begin("route")
+        tables = self._route(selected_experts, routing_weights, with_tiles=True)
+        tm.end()
+        tm.begin("fc1_swiglu")
+        act, fc1_out, fc1_scale = K.fc1_swiglu(
+            hidden_states, tables.send_token, gate_up_weight, tables.offsets, tables.weight_perm, num_routes,
+            self.activation, self.situ_beta, self.situ_linear_beta, self.clamp_limit, save_fc1=return_saved,
+            fc1_dtype=self.config.save_fc1_dtype, pool=self._workspaces, tiles=tables.tiles)
+        tm.end()
+        tm.begin("fc2")
+        se, sh, sf = down_weight.stride()
+        y = K.grouped_gemm(act, None, down_weight, se, sh, sf, tables.offsets, num_routes, self.hidden_size,
+                           inter, pool=self._workspaces, tiles=tables.tiles)
+        tm.end()
+        tm.begin("combine")
+        out = K.combine(y, tables.route_to_send, num_tokens, self.top_k)
+        tm.end()
+        return out, tables, act, fc1_out, fc1_scale
+
     def forward(self, hidden_states, selected_experts, gate_up_weight, down_weight, routing_weights, *,
                 return_saved: bool = False):
         """Run the complete BF16 post-routing MoE forward.
@@ -380,7 +409,7 @@ class FusedMoEForward(torch.nn.Module):
         """
         self._validate_dispatch_inputs(hidden_states, selected_experts)
         self._validate_gate_up_weight(gate_up_weight, hidden_states.device)
-        self._check_stream(hidden_states.device)
+        stream = self._check_stream(hidden_states.device)
         self._validate_routing_weights(routing_weights, selected_experts)
         self._validate_down_weight(down_weight, gate_up_weight, hidden_states.device)
         self._validate_tiles(gate_up_weight)
@@ -393,26 +422,18 @@ class FusedMoEForward(torch.nn.Module):
             out = torch.empty(0, self.hidden_size, dtype=torch.bfloat16, device=hidden_states.device)
             if not return_saved:
                 return out
-        tm = self.stage_timer or NULL_TIMER
         tables = None
-        if num_tokens:
-            tm.begin("route")
-            tables = self._route(selected_experts, routing_weights, with_tiles=True)
-            tm.end()
-            tm.begin("fc1_swiglu")
-            act, fc1_out, fc1_scale = K.fc1_swiglu(
-                hidden_states, tables.send_token, gate_up_weight, tables.offsets, tables.weight_perm, num_routes,
-                self.activation, self.situ_beta, self.situ_linear_beta, self.clamp_limit, save_fc1=return_saved,
-                fc1_dtype=self.config.save_fc1_dtype, pool=self._workspaces, tiles=tables.tiles)
-            tm.end()
-            tm.begin("fc2")
-            se, sh, sf = down_weight.stride()
-            y = K.grouped_gemm(act, None, down_weight, se, sh, sf, tables.offsets, num_routes, self.hidden_size,
-                               inter, pool=self._workspaces, tiles=tables.tiles)
-            tm.end()
-            tm.begin("combine")
-            out = K.combine(y, tables.route_to_send, num_tokens, self.top_k)
-            tm.end()
+        if num_tokens and self.stage_timer is None:
+            self._reserve_workspaces(hidden_states.device)
+            if return_saved:
+                tables = RouteTables(num_routes, self.experts_per_rank, self.top_k, hidden_states.device, True, True)
+            out, act, fc1_out, fc1_scale = K.layer_forward(
+                hidden_states, selected_experts, routing_weights, gate_up_weight, down_weight, self.experts_per_rank,
+                self.activation, self.situ_beta, self.situ_linear_beta, self.clamp_limit, tables,
+                self.config.save_fc1_dtype, stream.cuda_stream)
+        elif num_tokens:
+            out, tables, act, fc1_out, fc1_scale = self._forward_staged(
+                hidden_states, selected_experts, gate_up_weight, down_weight, routing_weights, return_saved)
         if not return_saved:
             return out
         saved = MoESaved(
