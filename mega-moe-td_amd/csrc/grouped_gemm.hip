@@ -172,7 +172,7 @@ __device__ __forceinline__ v4i16 lds_read_tr16(const bf16* p) {
 // row itself selects a quarter and swz = (r >> 2) & 3 separates the rest.
 // (Measured: FC1 bank-conflict cycles 2.7e7 -> 8.7e5.) Rows outside the tile
 // point at a valid row; their products are never stored.
-template <int ROWS, int BK_, int NT = kThreads>
+template <int ROWS, int BK_, int NT = kThreads, int KD = 16>
 struct KcTile {
   static constexpr int ELEMS = ROWS * BK_;
   static constexpr int VPR = BK_ / 8;                      // vectors per row
@@ -211,22 +211,32 @@ struct KcTile {
     for (int v = 0; v < PER_WAVE; ++v)
       *reinterpret_cast<u32x4_t*>(lds + (v * (NT / 64) + wave) * kChunkElems + lane * 8) = r[v];
   }
-  // MFMA 32x32x16 operand: row r0 + lane%32, k = kk + 8*(lane/32) .. +8
+  // MFMA operand of K depth KD: 32 rows x 16 (32x32x16: row r0 + lane % 32, k =
+  // kk + 8 * (lane / 32) .. + 8) or 16 rows x 32 (16x16x32, with 16 for 32)
   __device__ static bf16x8 frag(const bf16* lds, int r0, int kk, int lane) {
-    const int r = r0 + (lane & 31);
-    const int kv = (kk >> 3) + (lane >> 5);
+    constexpr int FR = KD == 32 ? 16 : 32;
+    const int r = r0 + (lane & (FR - 1));
+    const int kv = (kk >> 3) + lane / FR;
     return *reinterpret_cast<const bf16x8*>(lds + r * BK_ + ((kv ^ swz(r)) << 3));
   }
 };
 
 // Swizzle of the N-contiguous tile: vector slot of (k, source vector cv) is
-// cv ^ mn_swz(k). The pattern keeps the 4 K-rows x 32 bytes touched by a
-// 16-lane transposing read in distinct banks for 128- and 256-byte passes.
-__device__ __forceinline__ int mn_swz(int k) { return (0xEA40 >> ((k & 3) * 4)) & 0xF; }  // {0,4,10,14}
+// cv ^ mn_swz(k). KD is the K depth of the MFMA that reads the fragments.
+// 16 (32x32x16): a 32-lane pass takes 64 bytes of 4 K rows. 32 (16x16x32): it
+// takes 32 bytes of 8 K rows (0-3 and 8-11, then 16-19 and 24-27). Either
+// way the pieces of a pass sit in distinct banks.
+template <int KD>
+__device__ __forceinline__ int mn_swz(int k) {
+  if constexpr (KD == 32)
+    return ((k & 3) | ((k >> 1) & 4)) * 2;
+  else
+    return (0xEA40 >> ((k & 3) * 4)) & 0xF;  // {0,4,10,14}
+}
 
 // M/N-contiguous operand: LDS [BK_][ROWS] in the source's natural layout
 // (swizzled); MFMA fragments are read with the transposing LDS read.
-template <int ROWS, int BK_, int NT = kThreads>
+template <int ROWS, int BK_, int NT = kThreads, int KD = 16>
 struct MnTile {
   static constexpr int ELEMS = BK_ * ROWS;
   static constexpr int VPR = ROWS / 8;                      // 16-byte vectors per K row
@@ -234,11 +244,8 @@ struct MnTile {
   static constexpr int PER_WAVE = CHUNKS / (NT / 64);
   static constexpr int KPC = 64 / VPR;                      // K rows per 1 KiB chunk
   static_assert(PER_WAVE * (NT / 64) == CHUNKS, "chunks/waves mismatch");
-  static_assert(VPR >= 8, "swizzle needs >= 8 vectors per row");
+  static_assert(VPR >= 16, "swizzle needs >= 16 vectors per row");
   const bf16* ptr[PER_WAVE];
-
-  // 64-column rows: two rows per 64-bank line, so rows k and k + 2 swap halves
-  __device__ static int swz(int k) { return VPR >= 16 ? mn_swz(k) : ((k >> 1) & 1) * 4; }
 
   // K row and source column (elements) this lane copies in instruction v.
   __device__ static int k_of(int v) {
@@ -246,7 +253,7 @@ struct MnTile {
   }
   __device__ static int col_of(int v) {
     const int q = (v * (NT / 64) + (threadIdx.x >> 6)) * 64 + (threadIdx.x & 63);
-    return ((q % VPR) ^ swz(q / VPR)) * 8;
+    return ((q % VPR) ^ mn_swz<KD>(q / VPR)) * 8;
   }
   // Fixed-stride source: element (k, c) at base + k*ld + col_off(c).
   template <class ColOff>
@@ -279,12 +286,14 @@ struct MnTile {
     for (int v = 0; v < PER_WAVE; ++v)
       copy16_to_lds(src(v) + col_of(v), lds + (v * (NT / 64) + wave) * kChunkElems);
   }
+  // MFMA operand: 16 columns x 32 K rows (KD 32) or 32 x 16 (KD 16) from
+  // column r0, K row kk
   __device__ static bf16x8 frag(const bf16* lds, int r0, int kk, int lane) {
     const int s = lane & 15, g = lane >> 4;
-    const int k = kk + 8 * (g >> 1) + (s >> 2);
-    const int col = r0 + 16 * (g & 1) + 4 * (s & 3);
-    const bf16* q0 = lds + k * ROWS + ((((col >> 3) ^ swz(k)) << 3) | (col & 7));
-    const bf16* q1 = lds + (k + 4) * ROWS + ((((col >> 3) ^ swz(k + 4)) << 3) | (col & 7));
+    const int k = kk + 8 * (KD == 32 ? g : g >> 1) + (s >> 2);
+    const int col = r0 + (KD == 32 ? 0 : 16 * (g & 1)) + 4 * (s & 3);
+    const bf16* q0 = lds + k * ROWS + ((((col >> 3) ^ mn_swz<KD>(k)) << 3) | (col & 7));
+    const bf16* q1 = lds + (k + 4) * ROWS + ((((col >> 3) ^ mn_swz<KD>(k + 4)) << 3) | (col & 7));
     const v4i16 lo = lds_read_tr16(q0);
     const v4i16 hi = lds_read_tr16(q1);
     const v8i16 w = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -373,6 +382,42 @@ struct MmaTile {
   // TRANS layout: elements 4g .. 4g + 3 of a block sit in row lane % 32 and
   // columns acc_col(g, lane) .. + 3.
   __device__ static int acc_col(int g, int lane) { return g * 8 + (lane >> 5) * 4; }
+};
+
+// A (MI x 16) x (NJ x 16) sub-tile in v_mfma_f32_16x16x32_bf16 blocks, for the
+// weight-streaming tiles. With N(0, 1) operands a kernel that keeps the matrix
+// cores busy runs at the chip's power limit, and this shape moves half the
+// accumulator bytes per flop of 32x32x16: matrix instructions alone sustain
+// 2.05-2.09 PFLOP/s against 1.75 (zeros: 2.44 either way). The blocks are
+// walked in serpentine order, so consecutive instructions share an operand
+// (2.09 against 1.98 with both operands changing). Streaming tiles of 256
+// experts with 128 rows: 4197 -> 4147 us per forward. The 256 x 256 tiles keep
+// 32x32x16: there the copies of the operands bind, the clock that the shape
+// gains (1.77 -> 2.0 GHz) only waits for them (-3 to +4% per GEMM), and the
+// weight gradients' transposing reads need twice the addresses (+2 to +6%).
+// The operands are swapped, so acc[i][j] holds the transposed block: lane l
+// has the 4 consecutive columns 4 * (l / 16) of row l % 16.
+template <int MI, int NJ>
+struct MmaSlab {
+  f32x4 acc[MI][NJ];
+
+  __device__ void zero() {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  __device__ __forceinline__ void mfmas(const bf16x8 (&a)[MI], const bf16x8 (&b)[NJ]) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int q = 0; q < NJ; ++q) {
+        const int j = (i & 1) ? NJ - 1 - q : q;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+      }
+  }
+  // Column of a lane's 4 consecutive ones within a block (its row: lane % 16).
+  __device__ static int acc_col(int lane) { return (lane >> 4) * 4; }
 };
 
 // Non-temporal 16- and 8-byte stores of GEMM outputs. Measured against plain
@@ -783,9 +828,10 @@ __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
 // 1081; 60 experts of 68 rows, 2304 x 1792 109 -> 92.
 template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int ACT, int WN, int BPOL>
 struct StreamRows {
-  static constexpr int NT = 512, WAVES = NT / 64, WK = WAVES / WN, NJ = BN / WN / 32, SUB = BK_ / 16;
-  static_assert(WN * WK == WAVES && NJ * WN * 32 == BN && SUB % WK == 0, "wave split");
-  using BTile = typename std::conditional<BLAYOUT == B_KCONTIG, KcTile<BN, BK_, NT>, MnTile<BN, BK_, NT>>::type;
+  static constexpr int NT = 512, WAVES = NT / 64, WK = WAVES / WN, NJ = BN / WN / 16, SUB = BK_ / 32;
+  static_assert(WN * WK == WAVES && NJ * WN * 16 == BN && NJ % 2 == 0 && SUB % WK == 0, "wave split");
+  using BTile =
+      typename std::conditional<BLAYOUT == B_KCONTIG, KcTile<BN, BK_, NT, 32>, MnTile<BN, BK_, NT, 32>>::type;
   static constexpr int BM = kStreamRows;
   static constexpr int EPI_ROWS = 128;  // rows staged per epilogue pass
   using Out = StageOut<EPI_ROWS, BN, NT>;
@@ -852,17 +898,13 @@ struct StreamRows {
       lb.template issue<BPOL>(buf + AEL, s * b_step);
     };
     auto afrag = [&](const bf16* lds, int r0, int kk) {
-      const int r = r0 + (lane & 31), kv = (kk >> 3) + (lane >> 5);
+      const int r = r0 + (lane & 15), kv = (kk >> 3) + (lane >> 4);
       return *reinterpret_cast<const bf16x8*>(lds + r * BK_ + ((kv ^ a_swz(r)) << 3));
     };
 
-    f32x16 acc[MI][NJ];
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    using Mma = MmaSlab<2 * MI, NJ>;
+    Mma mma;
+    mma.zero();
     const int nk = p.k / BK_;
 #pragma unroll
     for (int s = 0; s < NST - 1; ++s)
@@ -875,84 +917,68 @@ struct StreamRows {
       const bf16* bs = as + AEL;
 #pragma unroll
       for (int t = 0; t < SUB / WK; ++t) {
-        const int kk = (t * WK + wk) * 16;
-        bf16x8 a[MI], b[NJ];
+        const int kk = (t * WK + wk) * 32;
+        bf16x8 a[2 * MI], b[NJ];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) b[j] = BTile::frag(bs, wn * (BN / WN) + j * 32, kk, lane);
+        for (int j = 0; j < NJ; ++j) b[j] = BTile::frag(bs, wn * (BN / WN) + j * 16, kk, lane);
 #pragma unroll
-        for (int i = 0; i < MI; ++i) a[i] = afrag(as, i * 32, kk);
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)  // operands swapped: a lane holds 4 consecutive columns of one row
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < 2 * MI; ++i) a[i] = afrag(as, i * 16, kk);
+        mma.mfmas(a, b);
       }
     }
     __syncthreads();
     if constexpr (WK > 1) {
-      float* red = reinterpret_cast<float*>(smem);  // [WK - 1][WN][NJ][16][64]
+      f32x4* red = reinterpret_cast<f32x4*>(smem);  // one slab: [WK - 1][WN][2][NJ][64]
 #pragma unroll
-      for (int i = 0; i < MI; ++i) {
+      for (int i = 0; i < 2 * MI; i += 2) {
         if (wk > 0) {
 #pragma unroll
-          for (int j = 0; j < NJ; ++j)
+          for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int r = 0; r < 16; r += 4)
-              *reinterpret_cast<f32x4*>(red + (((((wk - 1) * WN + wn) * NJ + j) * 4 + r / 4) * 64 + lane) * 4) =
-                  f32x4{acc[i][j][r], acc[i][j][r + 1], acc[i][j][r + 2], acc[i][j][r + 3]};
+            for (int j = 0; j < NJ; ++j) red[((((wk - 1) * WN + wn) * 2 + h) * NJ + j) * 64 + lane] = mma.acc[i + h][j];
         }
         __syncthreads();
         if (wk == 0) {
 #pragma unroll
           for (int w = 0; w < WK - 1; ++w)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-              for (int r = 0; r < 16; r += 4) {
-                const f32x4 v =
-                    *reinterpret_cast<const f32x4*>(red + ((((w * WN + wn) * NJ + j) * 4 + r / 4) * 64 + lane) * 4);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) acc[i][j][r + q] += v[q];
-              }
+              for (int j = 0; j < NJ; ++j) mma.acc[i + h][j] += red[(((w * WN + wn) * 2 + h) * NJ + j) * 64 + lane];
         }
         __syncthreads();
       }
     }
-    // epilogue: as rows_epilogue, with the columns split over the waves, in
-    // passes of at most EPI_ROWS rows
-    using Mma = MmaTile<32, 32, 1, 1>;
-    constexpr int PASS = EPI_ROWS / 32;
+    // in passes of at most EPI_ROWS rows
+    epilogue<MI, 0>(p, smem, mma, row0, rows, nt, wk, wn, lane, w_pre);
+    if constexpr (MI * 32 > EPI_ROWS) {
+      __syncthreads();  // the first pass has left LDS
+      epilogue<MI, EPI_ROWS / 32>(p, smem, mma, row0, rows, nt, wk, wn, lane, w_pre);
+    }
+  }
+
+  // As rows_epilogue, with the columns split over the waves, for slabs I0 ..
+  template <int MI, int I0, class Mma, int EPI_IT>
+  __device__ __forceinline__ static void epilogue(const RowsArgs& p, bf16* smem, const Mma& mma, int row0, int rows,
+                                                  int nt, int wk, int wn, int lane, const float (&w_pre)[EPI_IT]) {
+    constexpr int NS = (MI - I0 < EPI_ROWS / 32 ? MI - I0 : EPI_ROWS / 32), ER = NS * 32;
+    if (wk == 0) {
 #pragma unroll
-    for (int i0 = 0; i0 < MI; i0 += PASS) {
-      constexpr int LAST = MI % PASS == 0 ? PASS : MI % PASS;  // slabs of the last pass
-      if (i0 > 0) __syncthreads();                             // the previous pass has left LDS
-      if (wk == 0) {
+      for (int i = 0; i < 2 * NS; ++i)
 #pragma unroll
-        for (int i = i0; i < min(MI, i0 + PASS); ++i)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) {
-            const int g = wn * NJ + j;  // 32-column group of the tile
-            const int c0 = EPI == EPI_GATED ? (g & 1) * (BN / 2) + (g >> 1) * 32 : g * 32;
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-              Out::put4(smem, (i - i0) * 32 + (lane & 31), c0 + Mma::acc_col(q, lane), acc[i][j][4 * q],
-                        acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-          }
-      }
-      const int r0 = row0 + i0 * 32, nr = rows - i0 * 32;
-      auto w_of = [&](int it) { return w_pre[i0 * 32 * EPI_VPR / NT + it]; };
-      if constexpr (EPI == EPI_STORE) {
-        if (i0 + PASS < MI)
-          Out::flush(smem, min(nr, EPI_ROWS), p.c + static_cast<int64_t>(r0) * p.ldc + nt * BN, p.ldc);
-        else
-          StageOut<LAST * 32, BN, NT>::flush(smem, nr, p.c + static_cast<int64_t>(r0) * p.ldc + nt * BN, p.ldc);
-      } else {
-        __syncthreads();
-        if (i0 + PASS < MI)
-          gated_store<EPI_ROWS, BN, NT, ACT>(p, smem, r0, min(nr, EPI_ROWS), nt, w_of);
-        else
-          gated_store<LAST * 32, BN, NT, ACT>(p, smem, r0, nr, nt, w_of);
-      }
+        for (int j = 0; j < NJ; ++j) {
+          const int g = (wn * NJ + j) >> 1;  // 32-column group of the tile
+          const int c0 = (EPI == EPI_GATED ? (g & 1) * (BN / 2) + (g >> 1) * 32 : g * 32) + (j & 1) * 16;
+          const f32x4 c = mma.acc[2 * I0 + i][j];
+          Out::put4(smem, i * 16 + (lane & 15), c0 + Mma::acc_col(lane), c[0], c[1], c[2], c[3]);
+        }
+    }
+    const int r0 = row0 + I0 * 32, nr = min(rows - I0 * 32, ER);
+    if constexpr (EPI == EPI_STORE) {
+      StageOut<ER, BN, NT>::flush(smem, nr, p.c + static_cast<int64_t>(r0) * p.ldc + nt * BN, p.ldc);
+    } else {
+      __syncthreads();
+      gated_store<ER, BN, NT, ACT>(p, smem, r0, nr, nt, [&](int it) { return w_pre[I0 * 32 * (BN / 16) / NT + it]; });
     }
   }
 };
@@ -1196,7 +1222,7 @@ __global__ __launch_bounds__(NT) void wgrad_reg_kernel(WgradArgs a, int num_expe
     const int kg = r0 + s * BK_ + kl;            // row of the expert-major order
     const int lo = __builtin_amdgcn_readlane(ids, v * KPC), hi = __builtin_amdgcn_readlane(ids, v * KPC + 1);
     const int row = rows ? (half ? hi : lo) : min(kg, cap1);
-    const int c = (lcol ^ mn_swz(kl)) * 8;
+    const int c = (lcol ^ mn_swz<16>(kl)) * 8;
     const uint64_t data = reinterpret_cast<uint64_t>(base + static_cast<int64_t>(row) * ld + col0 + c);
     const uint64_t zero = reinterpret_cast<uint64_t>(g_wgrad_zero_row + c);
     const uint64_t addr = (zero_tail && kg >= r1) ? zero : data;
