@@ -1366,7 +1366,7 @@ __device__ __forceinline__ void wait_vmcnt_atmost(int n) {
 //    mod 8) owns a fixed subset of the experts: every expert writes the same
 //    n1 x n2 output whatever its row count, so this is balanced, and an
 //    expert's rows are read into that XCD's L2 once. A team of the XCD's
-//    workgroups takes every nc-th tile of its expert.
+//    workgroups takes every nc-th tile of its experts' tiles.
 //  * The product is formed transposed, C^T = Q^T P, so each lane's
 //    accumulator holds 4 consecutive output columns of one output row; every
 //    wave stages its 64 x 128 sub-tile 64 columns at a time in a private LDS
@@ -1392,10 +1392,13 @@ struct TileCursor {
     kr = min(o.y, rows_cap) - r0;
     nk = kr > 0 ? (kr + 31) / 32 : 1;  // an expert without rows still writes its zero tiles
   }
-  __device__ void skip_empty(int c, int per_e, int E, const int32_t* offsets, int rows_cap) {
+  // t runs on across the cursor's experts, so that a team whose size does not
+  // divide an expert's tiles leaves no workgroup idle at each expert's end
+  // (128 experts of 24 tiles over teams of 16: 150 -> 127 us)
+  __device__ void next_expert(int per_e, int E, const int32_t* offsets, int rows_cap) {
     while (valid && t >= per_e) {
       e += estep;
-      t = c;
+      t -= per_e;
       valid = e < E;
     }
     if (valid) load_expert(offsets, rows_cap);
@@ -1406,13 +1409,13 @@ struct TileCursor {
     t = c;
     ks = 0;
     valid = e < E;
-    skip_empty(c, per_e, E, offsets, rows_cap);
+    next_expert(per_e, E, offsets, rows_cap);
   }
-  __device__ void advance(int c, int nc, int per_e, int E, const int32_t* offsets, int rows_cap) {
+  __device__ void advance(int nc, int per_e, int E, const int32_t* offsets, int rows_cap) {
     if (++ks < nk) return;
     ks = 0;
     t += nc;
-    if (t >= per_e) skip_empty(c, per_e, E, offsets, rows_cap);
+    if (t >= per_e) next_expert(per_e, E, offsets, rows_cap);
   }
 };
 
@@ -1430,13 +1433,20 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
   constexpr int SPT = HALVES * SUB / 8 / 64;              // stores per lane per tile
   __shared__ __attribute__((aligned(1024))) bf16 smem[NST * STAGE + (NT / 64) * SUB];
   // Each XCD's workgroups form two teams (one if their count is odd), each
-  // walking its own expert: team q of XCD x0 takes experts x0 + 8q,
+  // walking its own experts: team q of XCD x0 takes experts x0 + 8q,
   // x0 + 8q + 8 * teams, ... (16 workgroups per expert measured 2% faster
-  // than 32 on the Kimi-scale gradients, and 4 teams no faster than 2).
+  // than 32 on the Kimi-scale gradients, and 4 teams no faster than 2). With
+  // fewer experts than teams the whole grid is one team, if that gives every
+  // workgroup tiles to walk.
   const int per_xcd = gridDim.x / kXcds;
   const int teams = per_xcd % 2 == 0 ? 2 : 1;
   const int team = (blockIdx.x / kXcds) % teams;
-  const int x = blockIdx.x % kXcds + team * kXcds, c = blockIdx.x / kXcds / teams, nc = per_xcd / teams;
+  const bool one_team = num_experts < kXcds * teams &&
+                        num_experts * (a.n1 / BM) * (a.n2 / BN) > 2 * static_cast<int>(gridDim.x);
+  const int x = one_team ? 0 : blockIdx.x % kXcds + team * kXcds;
+  const int c = one_team ? blockIdx.x : blockIdx.x / kXcds / teams;
+  const int nc = one_team ? gridDim.x : per_xcd / teams;
+  const int estep = one_team ? 1 : kXcds * teams;
   const int t1n = a.n1 / BM, t2n = a.n2 / BN;
   const int per_e = t1n * t2n;
   // Tile t of an expert -> (t1, t2): the dimension with more tiles varies
@@ -1461,7 +1471,7 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
   bf16* stage_out = smem + NST * STAGE + wave * SUB;
 
   TileCursor cc, lc;  // consumer; copier (NST - 1 stages ahead)
-  cc.init(x, kXcds * teams, c, per_e, num_experts, a.offsets, a.rows_cap);
+  cc.init(x, estep, c, per_e, num_experts, a.offsets, a.rows_cap);
   lc = cc;
   // Gathered operands: instruction v of this wave copies the stage's K rows
   // k0(v) .. k0(v) + KPC - 1 (k0 wave-uniform), so their row ids come from
@@ -1543,7 +1553,7 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
 #pragma unroll
     for (int i = 0; i < NST; ++i)
       if (i == nissued % NST) stage_mark[i] = issued_ops;
-    lc.advance(c, nc, per_e, num_experts, a.offsets, a.rows_cap);
+    lc.advance(nc, per_e, num_experts, a.offsets, a.rows_cap);
     if (lc.valid) load_ids(lc);
   }
   Mma mma;
@@ -1561,7 +1571,7 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
 #pragma unroll
       for (int i = 0; i < NST; ++i)
         if (i == nissued % NST) stage_mark[i] = issued_ops;
-      lc.advance(c, nc, per_e, num_experts, a.offsets, a.rows_cap);
+      lc.advance(nc, per_e, num_experts, a.offsets, a.rows_cap);
       if (lc.valid) load_ids(lc);
       ++nissued;
     }
@@ -1601,7 +1611,7 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
       issued_ops += SPT;
       mma.zero();
     }
-    cc.advance(c, nc, per_e, num_experts, a.offsets, a.rows_cap);
+    cc.advance(nc, per_e, num_experts, a.offsets, a.rows_cap);
   }
 }
 
