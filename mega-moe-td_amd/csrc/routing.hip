@@ -12,8 +12,9 @@
 // and one 16-wavefront workgroup. A workgroup needs, per expert, the routes in
 // earlier units and in all units; mostly it counts them itself from the ids
 // (L2-resident), so routing is ONE launch; else a first launch writes
-// unit_counts[unit][expert] and every workgroup sums the table (see
-// recount_routes). A block scan over the experts then gives every expert's
+// unit_counts[unit][expert], and every workgroup sums the table or a second
+// launch scans it (see units_source). A block scan over the experts then
+// gives every expert's
 // first row, and each wavefront scatters its own 128 routes in order: a
 // route's rank among equal experts comes from ballot match masks, the running
 // counter per (wavefront, expert) sits in LDS, so the scatter is
@@ -137,12 +138,16 @@ __device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t* part) {
   return v + base;
 }
 
-// One workgroup per unit, E <= kFusedExperts. unit_counts: null (count all
-// routes here) or the [nunits][E] table of route_count_kernel.
+// Where a unit's workgroup gets the routes of the other units from: it counts
+// them itself, it sums the [nunits][E] table of route_count_kernel, or
+// route_scan_kernel has turned that table into the unit's first rows.
+enum { UNITS_RECOUNT = 0, UNITS_TABLE = 1, UNITS_SCANNED = 2 };
+
+// One workgroup per unit, E <= kFusedExperts.
 __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
-    const int32_t* __restrict__ sel, int64_t R, int top_k, int E, int nbits, int nunits,
-    const int32_t* __restrict__ unit_counts, const float* __restrict__ rw, int32_t* __restrict__ counts,
-    int32_t* __restrict__ offsets, int32_t* __restrict__ send_route, int32_t* __restrict__ send_token,
+    const int32_t* __restrict__ sel, int64_t R, int top_k, int E, int nbits, int nunits, int source,
+    const int32_t* __restrict__ unit_counts, const float* __restrict__ rw, int32_t* counts, int32_t* offsets,
+    int32_t* __restrict__ send_route, int32_t* __restrict__ send_token,
     int32_t* __restrict__ route_to_send, float* __restrict__ weight_perm, TileList* __restrict__ tlS,
     TileList* __restrict__ tl256) {
   __shared__ int seg[kFusedWaves * kFusedExperts];  // [wave][expert]: routes of the segment, then its next row
@@ -167,7 +172,9 @@ __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
     key[it] = route_valid(e, E) ? e : E;
     if (key[it] < E) atomicAdd(&seg[wave * E + key[it]], 1);
   }
-  if (unit_counts) {
+  if (source == UNITS_SCANNED) {
+    for (int e = tid; e < E; e += kFusedThreads) before[e] = unit_counts[static_cast<int64_t>(u) * E + e];
+  } else if (source == UNITS_TABLE) {
     for (int i = tid; i < nunits * E; i += kFusedThreads) {
       const int v = i / E, e = i - v * E;
       const int c = unit_counts[i];
@@ -207,8 +214,16 @@ __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
     }
     total = run + rest[tid];
   }
-  const int first = static_cast<int>(block_scan(static_cast<uint64_t>(total), part)) - total;
-  if (tid < E) {
+  int first = 0;
+  if (source == UNITS_SCANNED) {  // the rows are absolute, counts and offsets written
+    if (tid < E) {
+      first = offsets[tid];
+      total = counts[tid];
+    }
+  } else {
+    first = static_cast<int>(block_scan(static_cast<uint64_t>(total), part)) - total;
+  }
+  if (tid < E && source != UNITS_SCANNED) {
 #pragma unroll
     for (int w = 0; w < kFusedWaves; ++w) seg[w * E + tid] += first;
     if (u == 0) {
@@ -318,13 +333,19 @@ extern "C" size_t mm_route_workspace_bytes(int64_t num_routes, int32_t num_exper
 
 namespace {
 
-// Whether every unit counts the other units' routes itself instead of
-// summing a table that a first launch writes. Recounting costs each workgroup
-// R ids, the table its R / 2048 * E entries and a launch; measured (us,
-// recount / table): 65536 routes 14.3 / 13.1 over 128 experts and 15.9 / 23.9
-// over 896; 131072 routes over 32 experts 21.7 / 12.8. At 32768 routes and
-// below the launch alone costs more (11.2 over 32 experts, all of it).
-bool recount_routes(int64_t num_routes, int E) { return num_routes <= 32768 || E >= 512; }
+// Recounting costs each workgroup R ids, the table its R / 2048 * E entries
+// and a launch; measured (us, recount / table): 65536 routes 14.3 / 13.1 over
+// 128 experts and 15.9 / 23.9 over 896; 131072 routes over 32 experts 21.7 /
+// 12.8. At 32768 routes and below the launch alone costs more (11.2 over 32
+// experts, all of it). Both grow with the square of R, the scan does not: it
+// takes over at 2e8 ids or entries over all units (524288 routes over 600
+// experts, 1.3e8: 58 us recounted against 77 with a scan; 1048576 over 896,
+// 5.4e8: 191 against 153; 1048576 over 32, 8.4e6: 42 against 96).
+int units_source(int64_t num_routes, int E, int64_t nunits) {
+  const bool recount = num_routes <= 32768 || E >= 512;
+  if (nunits * (recount ? num_routes : nunits * E) > 200000000) return UNITS_SCANNED;
+  return recount ? UNITS_RECOUNT : UNITS_TABLE;
+}
 
 int route_launch(const int32_t* selected, int64_t num_routes, int32_t top_k, int32_t num_experts,
                  const float* routing_weights, int32_t* counts, int32_t* offsets, int32_t* send_route,
@@ -336,12 +357,14 @@ int route_launch(const int32_t* selected, int64_t num_routes, int32_t top_k, int
   TileList* tlS = tiles ? mm_tile_list_of(tiles, num_routes, E, kStreamRows) : nullptr;
   TileList* tl256 = tiles ? mm_tile_list_of(tiles, num_routes, E, 256) : nullptr;
   if (E <= kFusedExperts) {
-    const bool recount = recount_routes(num_routes, E);
-    if (!recount)
+    const int source = units_source(num_routes, E, nunits);
+    if (source != UNITS_RECOUNT)
       route_count_kernel<<<nunits, kThreads, E * sizeof(int), s>>>(selected, num_routes, E, nunits, unit_counts);
+    if (source == UNITS_SCANNED)
+      route_scan_kernel<<<1, 1024, (E + 1024) * sizeof(int), s>>>(unit_counts, E, nunits, counts, offsets);
     route_fused_kernel<<<nunits > 0 ? nunits : 1, kFusedThreads, 0, s>>>(
-        selected, num_routes, top_k, E, nbits, nunits > 0 ? nunits : 1, recount ? nullptr : unit_counts,
-        routing_weights, counts, offsets, send_route, send_token, route_to_send, weight_perm, tlS, tl256);
+        selected, num_routes, top_k, E, nbits, nunits > 0 ? nunits : 1, source,
+        unit_counts, routing_weights, counts, offsets, send_route, send_token, route_to_send, weight_perm, tlS, tl256);
     return mm_check_launch(what);
   }
   // dynamic LDS above 64 KiB (up to 132 KiB at kMaxExperts); set once

@@ -1,6 +1,6 @@
 """Routing in one launch and the M-tile lists it writes (GPU): units of 2048
 routes, the switch above 32768 routes and below 512 experts from recounting
-in every workgroup to a count table, and the switch at 1024 experts to the large-expert kernels."""
+in every workgroup to a count table, from both to a scanned table, and the switch at 1024 experts to the large-expert kernels."""
 
 import numpy as np
 import pytest
@@ -23,6 +23,9 @@ CASES = [
     (32769, 1, 511, False),
     (32769, 1, 512, False),  # recounting again
     (8192, 16, 896, False),
+    (39900, 16, 600, False),   # 312 units: recounted; the next one is scanned
+    (41000, 16, 600, False),
+    (83000, 16, 500, True),    # 649 units: scanned instead of summed
     (300, 3, 1025, False),
 ]
 
