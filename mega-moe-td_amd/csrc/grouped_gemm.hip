@@ -1364,8 +1364,9 @@ __device__ __forceinline__ void wait_vmcnt_atmost(int n) {
 //    ring, so the first stages of the next tile are in flight while the
 //    current tile is staged and stored. Each XCD (workgroup ids congruent
 //    mod 8) owns a fixed subset of the experts: every expert writes the same
-//    n1 x n2 output whatever its row count, so this is balanced, and an
-//    expert's rows are read into that XCD's L2 once. A team of the XCD's
+//    n1 x n2 output whatever its row count, so this is balanced while the
+//    stores dominate, and an expert's rows are read into that XCD's L2 once
+//    (teams_uneven finds the rows for which it isn't balanced). A team of the XCD's
 //    workgroups takes every nc-th tile of its experts' tiles.
 //  * The product is formed transposed, C^T = Q^T P, so each lane's
 //    accumulator holds 4 consecutive output columns of one output row; every
@@ -1419,6 +1420,45 @@ struct TileCursor {
   }
 };
 
+// Whether nteams (8 or 16) teams of nc workgroups, team q walking experts
+// q, q + nteams, ..., take more than 5/4 of the time of one team of them all.
+// A tile costs its 32-row K steps and, for its store, about four more; a
+// team's slowest workgroup walks a tile of its longest expert (per round of
+// that expert's per_e tiles) and an even share of the rest. Each wave finds
+// the same answer from the offsets before its first copy (lane l sums experts
+// l, l + 64, ..., which are all of team l % nteams).
+// One team shares any split of the rows, but reads each expert's rows into
+// every XCD's L2. Measured, dW1, teams -> one team: even experts slower (100
+// of 8 x 6 tiles: 157 -> 165 us), Zipf-routed ones faster where the busiest
+// team has many tiles (64 of 16 x 12 tiles: 1286 -> 501 us) but not where the
+// longest expert's single round is the time (256 of 4 x 4: 329 -> 359 us).
+constexpr int kTileStoreSteps = 4;
+__device__ __forceinline__ bool teams_uneven(const int32_t* offsets, int E, int rows_cap, int nteams, int nc,
+                                             int per_e) {
+  int64_t sum = 0, longest = 0;
+  for (int e = threadIdx.x & 63; e < E; e += 64) {
+    const int rows = min(offsets[e + 1], rows_cap) - min(offsets[e], rows_cap);
+    const int64_t steps = (rows > 0 ? (rows - 1) / 32 + 1 : 1) + kTileStoreSteps;
+    sum += steps;
+    longest = max(longest, steps);
+  }
+  for (int d = 32; d >= nteams; d >>= 1) {
+    sum += __shfl_xor(sum, d);
+    longest = max(longest, static_cast<int64_t>(__shfl_xor(longest, d)));
+  }
+  // both in steps x workgroups of the walk
+  auto cost = [&](int64_t all, int64_t most, int wgs) {
+    return most * ((per_e + wgs - 1) / wgs) * wgs + (all - most) * per_e;
+  };
+  int64_t busiest = cost(sum, longest, nc);
+  for (int d = nteams >> 1; d > 0; d >>= 1) {
+    busiest = max(busiest, static_cast<int64_t>(__shfl_xor(busiest, d)));
+    longest = max(longest, static_cast<int64_t>(__shfl_xor(longest, d)));
+    sum += __shfl_xor(sum, d);
+  }
+  return __builtin_amdgcn_readfirstlane(4 * nteams * busiest > 5 * cost(sum, longest, nc * nteams));
+}
+
 template <int NST>
 __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num_experts) {
   constexpr int BM = 256, BN = 256, BKS = 32, WM = 2, WN = 4, NT = WM * WN * 64;
@@ -1436,13 +1476,14 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
   // walking its own experts: team q of XCD x0 takes experts x0 + 8q,
   // x0 + 8q + 8 * teams, ... (16 workgroups per expert measured 2% faster
   // than 32 on the Kimi-scale gradients, and 4 teams no faster than 2). With
-  // fewer experts than teams the whole grid is one team, if that gives every
-  // workgroup tiles to walk.
+  // fewer experts than teams, or rows that load the teams unevenly, the whole
+  // grid is one team, if that gives every workgroup tiles to walk.
   const int per_xcd = gridDim.x / kXcds;
   const int teams = per_xcd % 2 == 0 ? 2 : 1;
   const int team = (blockIdx.x / kXcds) % teams;
-  const bool one_team = num_experts < kXcds * teams &&
-                        num_experts * (a.n1 / BM) * (a.n2 / BN) > 2 * static_cast<int>(gridDim.x);
+  const bool one_team = num_experts * (a.n1 / BM) * (a.n2 / BN) > 2 * static_cast<int>(gridDim.x) &&
+                        (num_experts < kXcds * teams || teams_uneven(a.offsets, num_experts, a.rows_cap, kXcds * teams, per_xcd / teams,
+                                      (a.n1 / BM) * (a.n2 / BN)));
   const int x = one_team ? 0 : blockIdx.x % kXcds + team * kXcds;
   const int c = one_team ? blockIdx.x : blockIdx.x / kXcds / teams;
   const int nc = one_team ? gridDim.x : per_xcd / teams;
