@@ -816,20 +816,19 @@ __global__ __launch_bounds__(NT) void grouped_rows_kernel(RowsArgs p) {
 }
 
 // Weight-streaming row GEMM for tiles of at most 160 rows, bound by reading
-// the weights. 8 waves split the N columns (WN of them) and, where the tile
-// has fewer than eight 32-column groups, the 16-deep K sub-steps of a stage
-// (8 / WN ways; their partial sums meet in LDS before the epilogue), so every
-// weight fragment is read from LDS once, and all waves work whatever the row
-// count. The A rows are copied and multiplied in slabs of 32, one loop per
+// the weights. The 8 waves split the N columns (16, 32 or 64 each), so every
+// weight fragment is read from LDS once, all waves work whatever the row
+// count, and an element's products are summed over ascending K whatever the
+// tile: a token's bits do not depend on the size of the call. The A rows are copied and multiplied in slabs of 32, one loop per
 // slab count. Against 8 waves split 4 x 2 over 128 padded rows (us): 8
 // experts of one row, 2048 x 1536 (gate and up) 55 -> 17 and 768 x 2048 26 ->
 // 11; 117 experts of 2 rows 149 -> 116 and 69 -> 60; 256 experts' share of
 // 7168 x 4096 at 2 rows 1145 -> 976 (6.0 -> 7.0 TB/s), at 73 rows 1159 ->
 // 1081; 60 experts of 68 rows, 2304 x 1792 109 -> 92.
-template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int ACT, int WN, int BPOL>
+template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int ACT, int BPOL>
 struct StreamRows {
-  static constexpr int NT = 512, WAVES = NT / 64, WK = WAVES / WN, NJ = BN / WN / 16, SUB = BK_ / 32;
-  static_assert(WN * WK == WAVES && NJ * WN * 16 == BN && NJ % 2 == 0 && SUB % WK == 0, "wave split");
+  static constexpr int NT = 512, WAVES = NT / 64, NJ = BN / WAVES / 16, SUB = BK_ / 32;
+  static_assert(NJ * WAVES * 16 == BN, "wave split");
   using BTile =
       typename std::conditional<BLAYOUT == B_KCONTIG, KcTile<BN, BK_, NT, 32>, MnTile<BN, BK_, NT, 32>>::type;
   static constexpr int BM = kStreamRows;
@@ -837,9 +836,7 @@ struct StreamRows {
   using Out = StageOut<EPI_ROWS, BN, NT>;
   static constexpr int AVPR = BK_ / 8;  // 16-byte vectors per A row
   static constexpr int ring(int mi) { return NST * (mi * 32 * BK_ + BTile::ELEMS); }
-  static constexpr int RED = WK > 1 ? (WK - 1) * 32 * BN * 2 : 0;  // fp32 partials of one slab, in bf16 elements
-  static constexpr int max2(int a, int b) { return a > b ? a : b; }
-  static constexpr int SMEM = max2(max2(ring(BM / 32), Out::ELEMS), RED);
+  static constexpr int SMEM = ring(BM / 32) > Out::ELEMS ? ring(BM / 32) : Out::ELEMS;
 
   // as KcTile, for any row length
   __device__ static int a_swz(int r) { return AVPR == 4 ? ((r >> 2) & 3) : AVPR == 8 ? ((r >> 1) & 7) : (r & 15); }
@@ -852,7 +849,6 @@ struct StreamRows {
     constexpr int STAGE = AEL + BTile::ELEMS;
     constexpr int LPS = PA + BTile::PER_WAVE;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wn = wave % WN, wk = wave / WN;
     const bf16* bexp = p.b + static_cast<int64_t>(e) * p.b_se;
     // B tile column c -> global column: gated tiles alternate 32-column groups of gate and up
     auto bcol = [&](int c) -> int64_t {
@@ -916,63 +912,39 @@ struct StreamRows {
       const bf16* as = smem + (kt % NST) * STAGE;
       const bf16* bs = as + AEL;
 #pragma unroll
-      for (int t = 0; t < SUB / WK; ++t) {
-        const int kk = (t * WK + wk) * 32;
+      for (int t = 0; t < SUB; ++t) {
+        const int kk = t * 32;
         bf16x8 a[2 * MI], b[NJ];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) b[j] = BTile::frag(bs, wn * (BN / WN) + j * 16, kk, lane);
+        for (int j = 0; j < NJ; ++j) b[j] = BTile::frag(bs, (wave * NJ + j) * 16, kk, lane);
 #pragma unroll
         for (int i = 0; i < 2 * MI; ++i) a[i] = afrag(as, i * 16, kk);
         mma.mfmas(a, b);
       }
     }
     __syncthreads();
-    if constexpr (WK > 1) {
-      f32x4* red = reinterpret_cast<f32x4*>(smem);  // one slab: [WK - 1][WN][2][NJ][64]
-#pragma unroll
-      for (int i = 0; i < 2 * MI; i += 2) {
-        if (wk > 0) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) red[((((wk - 1) * WN + wn) * 2 + h) * NJ + j) * 64 + lane] = mma.acc[i + h][j];
-        }
-        __syncthreads();
-        if (wk == 0) {
-#pragma unroll
-          for (int w = 0; w < WK - 1; ++w)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-              for (int j = 0; j < NJ; ++j) mma.acc[i + h][j] += red[(((w * WN + wn) * 2 + h) * NJ + j) * 64 + lane];
-        }
-        __syncthreads();
-      }
-    }
     // in passes of at most EPI_ROWS rows
-    epilogue<MI, 0>(p, smem, mma, row0, rows, nt, wk, wn, lane, w_pre);
+    epilogue<MI, 0>(p, smem, mma, row0, rows, nt, wave, lane, w_pre);
     if constexpr (MI * 32 > EPI_ROWS) {
       __syncthreads();  // the first pass has left LDS
-      epilogue<MI, EPI_ROWS / 32>(p, smem, mma, row0, rows, nt, wk, wn, lane, w_pre);
+      epilogue<MI, EPI_ROWS / 32>(p, smem, mma, row0, rows, nt, wave, lane, w_pre);
     }
   }
 
   // As rows_epilogue, with the columns split over the waves, for slabs I0 ..
   template <int MI, int I0, class Mma, int EPI_IT>
   __device__ __forceinline__ static void epilogue(const RowsArgs& p, bf16* smem, const Mma& mma, int row0, int rows,
-                                                  int nt, int wk, int wn, int lane, const float (&w_pre)[EPI_IT]) {
+                                                  int nt, int wave, int lane, const float (&w_pre)[EPI_IT]) {
     constexpr int NS = (MI - I0 < EPI_ROWS / 32 ? MI - I0 : EPI_ROWS / 32), ER = NS * 32;
-    if (wk == 0) {
 #pragma unroll
-      for (int i = 0; i < 2 * NS; ++i)
+    for (int i = 0; i < 2 * NS; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const int g = (wn * NJ + j) >> 1;  // 32-column group of the tile
-          const int c0 = (EPI == EPI_GATED ? (g & 1) * (BN / 2) + (g >> 1) * 32 : g * 32) + (j & 1) * 16;
-          const f32x4 c = mma.acc[2 * I0 + i][j];
-          Out::put4(smem, i * 16 + (lane & 15), c0 + Mma::acc_col(lane), c[0], c[1], c[2], c[3]);
-        }
-    }
+      for (int j = 0; j < NJ; ++j) {
+        const int b = wave * NJ + j, g = b >> 1;  // 16-column block, its 32-column group of the tile
+        const int c0 = (EPI == EPI_GATED ? (g & 1) * (BN / 2) + (g >> 1) * 32 : g * 32) + (b & 1) * 16;
+        const f32x4 c = mma.acc[2 * I0 + i][j];
+        Out::put4(smem, i * 16 + (lane & 15), c0 + Mma::acc_col(lane), c[0], c[1], c[2], c[3]);
+      }
     const int r0 = row0 + I0 * 32, nr = min(rows - I0 * 32, ER);
     if constexpr (EPI == EPI_STORE) {
       StageOut<ER, BN, NT>::flush(smem, nr, p.c + static_cast<int64_t>(r0) * p.ldc + nt * BN, p.ldc);
@@ -983,9 +955,9 @@ struct StreamRows {
   }
 };
 
-template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int ACT, int WN, int BPOL>
+template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int ACT, int BPOL>
 __global__ __launch_bounds__(512) void stream_rows_kernel(RowsArgs p) {
-  using K = StreamRows<BN, BK_, NST, BLAYOUT, EPI, ACT, WN, BPOL>;
+  using K = StreamRows<BN, BK_, NST, BLAYOUT, EPI, ACT, BPOL>;
   __shared__ __attribute__((aligned(1024))) bf16 smem[K::SMEM];
   const int num_n = p.n / BN;
   const int num_m = p.tl->count;
@@ -1707,7 +1679,7 @@ void launch_rows_cfg(const RowsArgs& p, int64_t max_rows, int E, hipStream_t s) 
     grouped_rows_kernel<BM, BN, BK_, NST, BLAYOUT, EPI, NT, 0, REG><<<grid, NT, 0, s>>>(p);
 }
 
-template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int WN, int BPOL>
+template <int BN, int BK_, int NST, int BLAYOUT, int EPI, int BPOL>
 void launch_stream(RowsArgs p, int64_t max_rows, int E, hipStream_t s) {
   const int64_t mm = mm_max_m_tiles(max_rows, E, kStreamRows), num_n = p.n / BN;
   // Enough M tiles to even out over the XCDs: M tile m on XCD m % 8, its N
@@ -1724,10 +1696,10 @@ void launch_stream(RowsArgs p, int64_t max_rows, int E, hipStream_t s) {
   const int grid = static_cast<int>((g + kXcds - 1) / kXcds * kXcds);
   if constexpr (EPI == EPI_GATED)
     by_act(p.act_kind, [&](auto act) {
-      stream_rows_kernel<BN, BK_, NST, BLAYOUT, EPI, decltype(act)::value, WN, BPOL><<<grid, 512, 0, s>>>(p);
+      stream_rows_kernel<BN, BK_, NST, BLAYOUT, EPI, decltype(act)::value, BPOL><<<grid, 512, 0, s>>>(p);
     });
   else
-    stream_rows_kernel<BN, BK_, NST, BLAYOUT, EPI, 0, WN, BPOL><<<grid, 512, 0, s>>>(p);
+    stream_rows_kernel<BN, BK_, NST, BLAYOUT, EPI, 0, BPOL><<<grid, 512, 0, s>>>(p);
 }
 
 // 256x256 row tiles with K >= 1024: 4 waves of 128x128 with register-staged
@@ -1749,9 +1721,12 @@ bool rows_lds_dma() {
 // * factor is taken, for the experts that this many routes reach on average.
 // K-contiguous weights never take 512 (its 32-deep stages read 64-byte pieces
 // of every weight row: 3.7 against 6.5 TB/s). Measured, gate and up weights,
-// us at 512 / 256 / 128 columns: 8 experts of 2048 x 1536 45 / 24 / 17; 31:
-// 51 / 37 / 44; 56: 60 / 68 / 63; 112: 125 / 111 / 123; 14 experts of 4096 x
-// 3072 96 / 68 / 88; 32: 125 / 142 / 147.
+// one row per expert, us at 512 / 256 / 128 columns: 8 experts of 2048 x 1536
+// 41 / 23 / 18; 31: 50 / 35 / 41; 56: 59 / 69 / 62; 112: 124 / 110 / 121; 14
+// experts of 4096 x 3072 98 / 65 / 83; 32: 126 / 143 / 142.
+// (128 columns with K split over two waves instead of 16 columns for each:
+// within 1 us of these up to 14 experts, but its sums had another order than
+// the other tiles', so a token's bits changed with the size of the call.)
 // The weights are read once: their copies carry the non-temporal hint, which
 // keeps them from displacing the activation rows that the expert's N tiles
 // share (112 experts of 2048 x 1536: 111 against 124 us), unless all weights
@@ -1772,8 +1747,7 @@ StreamCfg pick_stream_cfg(int64_t max_rows, int E, int n, int k, bool n_contig, 
   StreamCfg c{128, false};
   double best = cost(128, 1.5);
   // a call that saves FC1 takes at least 256 columns: an FP8 save needs whole
-  // 128-column scale groups, and every format then narrows the same fp32 sums
-  // (128 columns split K over two waves, which sums in another order)
+  // 128-column scale groups
   if (n % 256 == 0 && (save || cost(256, 1.15) <= best)) {
     c.bn = 256;
     best = cost(256, 1.15);
@@ -1843,18 +1817,18 @@ int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const 
     const StreamCfg c = pick_stream_cfg(max_rows, E, p.n, p.k, BLAYOUT == B_NCONTIG, p.fc1_out != nullptr);
     if constexpr (BLAYOUT == B_NCONTIG) {
       if (c.bn == 512) {
-        launch_stream<512, 32, 3, BLAYOUT, EPI, 8, 1>(p, max_rows, E, s);
+        launch_stream<512, 32, 3, BLAYOUT, EPI, 1>(p, max_rows, E, s);
         return mm_check_launch(what);
       }
     }
     if (c.bn == 256 && c.nt)
-      launch_stream<256, 64, 3, BLAYOUT, EPI, 8, 1>(p, max_rows, E, s);
+      launch_stream<256, 64, 3, BLAYOUT, EPI, 1>(p, max_rows, E, s);
     else if (c.bn == 256)
-      launch_stream<256, 64, 3, BLAYOUT, EPI, 8, 0>(p, max_rows, E, s);
+      launch_stream<256, 64, 3, BLAYOUT, EPI, 0>(p, max_rows, E, s);
     else if (c.nt)
-      launch_stream<128, 64, 4, BLAYOUT, EPI, 4, 1>(p, max_rows, E, s);
+      launch_stream<128, 64, 4, BLAYOUT, EPI, 1>(p, max_rows, E, s);
     else
-      launch_stream<128, 64, 4, BLAYOUT, EPI, 4, 0>(p, max_rows, E, s);
+      launch_stream<128, 64, 4, BLAYOUT, EPI, 0>(p, max_rows, E, s);
   }
   return mm_check_launch(what);
 }
