@@ -1144,9 +1144,11 @@ __device__ __attribute__((aligned(256))) bf16 g_wgrad_zero_row[256];  // never w
 // copies are ordinary loads, so the compiler's own wait counts cover them.
 // Wave w copies the stage's K rows 16w .. 16w + 15 (two per 1 KiB chunk);
 // the row ids of a gathered operand arrive one stage earlier, one load per
-// wave (lanes 0..15), and are broadcast with readlane. P rows past the
-// expert's end are read from a zero row (their products vanish), Q rows
-// there from a clamped real row, so the loop body has no branch. The
+// wave (lanes 0..15), and are broadcast with readlane. Rows of both operands
+// past the expert's end are read from a zero row, so the loop body has no
+// branch: the row there may be another expert's or, past the last expert of
+// a call with dropped routes, one that was never written, and a zero times an
+// infinity or a NaN is a NaN. The
 // epilogue stages the tile in the (then idle) ring, XOR-swizzled, and stores
 // 2 rows x 512 B per instruction.
 template <int NT = 256>
@@ -1188,8 +1190,7 @@ __global__ __launch_bounds__(NT) void wgrad_reg_kernel(WgradArgs a, int num_expe
     const int r = min(r0 + s * BK_ + wave * RPW + (lane & (RPW - 1)), cap1);
     return *(rows ? rows + r : a.offsets);
   };
-  auto src = [&](const bf16* base, int64_t ld, const int32_t* rows, int ids, int s, int v, int64_t col0,
-                 bool zero_tail) {
+  auto src = [&](const bf16* base, int64_t ld, const int32_t* rows, int ids, int s, int v, int64_t col0) {
     const int kl = wave * RPW + v * KPC + half;  // K row within the stage
     const int kg = r0 + s * BK_ + kl;            // row of the expert-major order
     const int lo = __builtin_amdgcn_readlane(ids, v * KPC), hi = __builtin_amdgcn_readlane(ids, v * KPC + 1);
@@ -1197,18 +1198,18 @@ __global__ __launch_bounds__(NT) void wgrad_reg_kernel(WgradArgs a, int num_expe
     const int c = (lcol ^ mn_swz<16>(kl)) * 8;
     const uint64_t data = reinterpret_cast<uint64_t>(base + static_cast<int64_t>(row) * ld + col0 + c);
     const uint64_t zero = reinterpret_cast<uint64_t>(g_wgrad_zero_row + c);
-    const uint64_t addr = (zero_tail && kg >= r1) ? zero : data;
+    const uint64_t addr = kg >= r1 ? zero : data;
     return *reinterpret_cast<const u32x4_t*>(addr);
   };
   u32x4_t ra[PW], rb[PW];
   int pid_cur = 0, qid_cur = 0, pid_nxt = 0, qid_nxt = 0;
   auto gload_p = [&](int s) {
 #pragma unroll
-    for (int v = 0; v < PW; ++v) ra[v] = src(a.p, a.ldp, a.p_rows, pid_cur, s, v, pc, true);
+    for (int v = 0; v < PW; ++v) ra[v] = src(a.p, a.ldp, a.p_rows, pid_cur, s, v, pc);
   };
   auto gload_q = [&](int s) {
 #pragma unroll
-    for (int v = 0; v < PW; ++v) rb[v] = src(a.q, a.ldq, a.q_rows, qid_cur, s, v, qc, false);
+    for (int v = 0; v < PW; ++v) rb[v] = src(a.q, a.ldq, a.q_rows, qid_cur, s, v, qc);
   };
   // chunk v of wave w sits at LDS chunk w * PW + v (rows 2 (w PW + v) + 0/1)
   auto put = [&](bf16* buf, const u32x4_t (&r)[PW]) {

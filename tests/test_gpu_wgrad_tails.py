@@ -1,0 +1,41 @@
+"""Weight gradients of ragged experts beside rows that hold infinities and NaN
+(GPU): the rows after an expert's last one, another expert's or, with dropped
+routes, never written, take no part in its gradient."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# rows per expert choose the kernel: persistent, 64-row K steps, register-staged
+@pytest.mark.parametrize("counts,n1,n2", [
+    ([70, 1, 33, 50], 512, 256), ([500, 333, 1, 800], 256, 512), ([500, 333], 128, 384),
+    ([2100, 2049, 2177, 2500], 256, 512),
+])
+@pytest.mark.parametrize("gather", [False, True])
+def test_rows_past_the_end(counts, n1, n2, gather):
+    from mega_moe.ops import _kernels as K
+
+    g = torch.Generator(device="cuda").manual_seed(sum(counts))
+    E = len(counts)
+    offs = torch.tensor([0] + counts, dtype=torch.int32).cumsum(0).int()
+    n, cap = int(offs[-1]), int(offs[-1]) + 100  # 100 capacity rows hold no route
+    p = torch.randn(cap, n1, generator=g, device="cuda").bfloat16()
+    q = torch.randn(cap, n2, generator=g, device="cuda").bfloat16()
+    rows = torch.randperm(cap, generator=g, device="cuda").int() if gather else None
+    prow = rows.long() if gather else torch.arange(cap, device="cuda")
+    for bad, lo, hi in ((float("nan"), n, cap), (float("inf"), int(offs[1]), int(offs[2]))):
+        p[prow[lo:hi]] = bad  # never-written rows; all of expert 1
+        q[lo:hi] = bad
+    c = K.grouped_wgrad(p, rows, q, None, offs.cuda(), n1, n2, max_rows=cap)
+    torch.cuda.synchronize()
+    for e in range(E):
+        r0, r1 = int(offs[e]), int(offs[e + 1])
+        if e == 1:
+            continue
+        pe, qe = p[prow[r0:r1]].float(), q[r0:r1].float()
+        ref, mag = pe.t() @ qe, pe.abs().t() @ qe.abs()
+        err = (c[e].float() - ref).abs()
+        # fp32 sums in two orders, one bf16 rounding
+        assert bool((err <= 2.0 ** -8 * ref.abs() + (r1 - r0) * 2.0 ** -23 * mag).all()), (e, counts[e])
