@@ -64,6 +64,24 @@ def _side_stream(device) -> torch.cuda.Stream:
     return st
 
 
+def _tile_lists(saved, offsets, num_routes):
+    """The M-tile lists the forward saved, or ``None`` where they may not be
+    those of these offsets: each row GEMM then cuts its own from ``offsets``.
+
+    The lists are a second copy of the row partition (and laid out by the
+    route capacity), while the other kernels read the offsets, which a caller
+    may replace, trim or edit. So they count only beside the very tensor they
+    were cut from, unchanged since, and at the same capacity. An inference
+    tensor records no changes."""
+    tiles, key = saved.get("_tiles"), saved.get("_tiles_key")
+    if tiles is None or key is None:
+        return None
+    cut_from, version, capacity = key
+    if cut_from is not offsets or offsets.is_inference() or offsets._version != version:
+        return None
+    return tiles if num_routes == capacity and tiles.device == offsets.device else None
+
+
 def _one_call(saved, dy, x, tiles) -> bool:
     """Whether the pass can go through ``mm_moe_backward``: the saved tensors
     as the forward wrote them, on one device. Anything else takes the staged
@@ -133,7 +151,7 @@ def moe_backward_triton(saved, dy, peer_mem=None, grad_transport=None, hidden_st
     tm.mark_pass()
     pool = saved.get("_workspaces")
     ws_rows = saved.get("_max_routes") or R
-    tiles = saved.get("_tiles")
+    tiles = _tile_lists(saved, offsets, R)
     side = _side_stream(dy.device) if overlap_act_bwd(R, offsets.numel() - 1) else None
     if side is None and tm is NULL_TIMER and _one_call(saved, dy, x, tiles):
         act = None if saved_recompute() else saved.get("swiglu_out_weighted")

@@ -453,7 +453,7 @@ class FusedMoEForward(torch.nn.Module):
                 expert_counts=tables.counts, split_size_cum_per_expert=tables.offsets,
                 send_route_indices=tables.send_route, send_token_indices=tables.send_token,
                 route_to_send=tables.route_to_send, recv_weights_sorted=tables.weight_perm,
-                fc1_output=fc1_out, swiglu_out_weighted=act, _tiles=tables.tiles,
+                fc1_output=fc1_out, swiglu_out_weighted=act, _tiles=tables.tiles, _tiles_key=tables.tiles_key(),
             )
             if saved_recompute():
                 # MOE_SAVED_RECOMPUTE=1 (reference kernels/mega_bwd.py:3208-3226): the backward

@@ -77,6 +77,11 @@ class RouteTables:
         self.tiles = (torch.empty(int(_lib.load().mm_tile_lists_size(num_routes, num_experts)), dtype=torch.uint8,
                                   device=device) if with_tiles else None)
 
+    def tiles_key(self):
+        """What ``tiles`` was cut from: the offsets, their version and the row
+        capacity (``None`` for inference tensors, which have no version)."""
+        return None if self.offsets.is_inference() else (self.offsets, self.offsets._version, self.num_routes)
+
 
 def route(selected_experts: torch.Tensor, num_experts: int, routing_weights: Optional[torch.Tensor],
           workspace: torch.Tensor, with_tiles: bool = False) -> RouteTables:

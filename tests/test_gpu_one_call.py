@@ -72,3 +72,20 @@ def test_changed_saves_take_the_staged_calls():
     saved["fc1_output"] = saved["fc1_output"].float()
     with pytest.raises(TypeError):
         mega_moe.moe_backward_triton(saved, inp["dy"])
+
+
+def test_replaced_offsets_are_read():
+    spec = CaseSpec("replaced", 300, 256, 128, 4, 2, "softmax_topk", True)
+    inp = make_inputs(spec, device="cuda", seed=5, weight_scale=0.1)
+    got = []
+    for drop_lists in (False, True):
+        _, saved = _op(spec, "bf16").forward(inp["x"], inp["selected"], inp["gate_up"], inp["down"], inp["rw"],
+                                             return_saved=True)
+        moved = saved["split_size_cum_per_expert"].clone()
+        moved[1] -= 1  # the first expert's last row counts as the second's
+        saved["split_size_cum_per_expert"] = moved
+        if drop_lists:
+            del saved["_tiles"]
+        got.append(mega_moe.moe_backward_triton(saved, inp["dy"]))
+    for k in GRADS:
+        assert torch.equal(got[0][k], got[1][k]), k
