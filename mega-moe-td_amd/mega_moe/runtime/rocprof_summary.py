@@ -8,8 +8,8 @@ GRBM_COUNT of a one-step run of the same configuration, plus the FETCH_SIZE /
 WRITE_SIZE directories of ``bench.py --calibrate-copy`` (five 1 GiB device
 copies), which give the bytes per counter unit. Kernels are assigned to the
 layer's stages from their launch order within each step (a step starts at
-the routing kernel); a stage's tile-list build and operand permutes belong
-to it.
+its first routing kernel); a stage's tile-list build and operand permutes
+belong to it, the two builds of a routing above 1024 experts to the routing.
 
     python -m mega_moe.runtime.rocprof_summary --trace DIR --fetch DIR --write DIR \
         --clock DIR --cal-fetch DIR --cal-write DIR --bench JSON --md OUT.md --json OUT.json
@@ -63,23 +63,34 @@ def dispatches(directory: str, counter: str | None = None):
 
 
 def split_steps(disp):
-    """Group the layer's own kernels into steps; each step starts at the
-    routing count kernel. Kernels before the first step (input generation)
-    are dropped."""
-    steps, cur = [], None
+    """Group the layer's own kernels into steps; each step starts at the first
+    routing kernel (a count, or the fused kernel alone) after another one.
+    Kernels before the first step (input generation) are dropped."""
+    steps, cur, routing = [], None, False
     for d in disp:
         n = short_name(d[1])
-        if "route_count_kernel" in n:
+        if not _is_layer_kernel(n):
+            continue
+        if _is_routing(n) and not routing:
             cur = []
             steps.append(cur)
-        if cur is not None and _is_layer_kernel(n):
+        routing = _is_routing(n)
+        if cur is not None:
             cur.append(d)
     return steps
 
 
+def _is_routing(n: str) -> bool:
+    return any(s in n for s in ("route_count_kernel", "route_scan_kernel", "route_fused_kernel", "route_scatter"))
+
+
+def _is_row_gemm(n: str) -> bool:
+    return "grouped_rows" in n or "stream_rows" in n
+
+
 def _is_layer_kernel(n: str) -> bool:
-    return any(s in n for s in ("route_", "build_tiles", "grouped_rows", "combine_items", "gather_route_grad",
-                                "swiglu_bwd", "gated_act", "permute_kernel", "wgrad"))
+    return _is_routing(n) or _is_row_gemm(n) or any(s in n for s in (
+        "build_tiles", "combine_items", "gather_route_grad", "swiglu_bwd", "gated_act", "permute_kernel", "wgrad"))
 
 
 def assign_stages(step):
@@ -88,17 +99,20 @@ def assign_stages(step):
     gemm_i = wgrad_i = 0
     combines = 0
     pending = []  # permutes waiting for their weight gradient
-    cur_gemm = None
+    lists = []  # tile-list builds waiting for their row GEMM
     for d in step:
         n = short_name(d[1])
-        if n.startswith("route_"):
+        if _is_routing(n):
             out.setdefault("route", []).append(d)
         elif "build_tiles" in n:
-            cur_gemm = GEMM_ORDER[gemm_i]
+            lists.append(d)
+        elif _is_row_gemm(n):
+            if len(lists) > 1:  # both lists of the pass, built by its routing
+                out.setdefault("route", []).extend(lists)
+                lists = []
+            out.setdefault(GEMM_ORDER[gemm_i], []).extend(lists + [d])
             gemm_i += 1
-            out.setdefault(cur_gemm, []).append(d)
-        elif "grouped_rows" in n:
-            out.setdefault(cur_gemm, []).append(d)
+            lists = []
         elif "combine_items" in n:
             out.setdefault("combine" if combines == 0 else "combine_bwd", []).append(d)
             combines += 1
@@ -163,7 +177,7 @@ def mfma_table(pmc_dir: str, bench: dict, title: str) -> str:
     for stage, ds in assign_stages(step).items():
         if stage not in GEMM_LABELS:
             continue
-        main_k = [d for d in ds if "grouped_rows" in d[1] or "wgrad" in d[1]]
+        main_k = [d for d in ds if _is_row_gemm(d[1]) or "wgrad" in d[1]]
         if not main_k:
             continue
         d = main_k[-1]

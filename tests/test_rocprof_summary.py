@@ -6,6 +6,8 @@ import csv
 import json
 import os
 
+import pytest
+
 from mega_moe.runtime import rocprof_summary as R
 
 STEP = [  # one fwd+bwd step, launch order, (kernel name, duration ns)
@@ -100,3 +102,47 @@ def test_overlap_note_for_stage_without_bench_time(tmp_path):
             "--cal-fetch", str(tmp_path / "cf"), "--cal-write", str(tmp_path / "cw"), "--bench",
             str(tmp_path / "b.json"), "--md", md])
     assert "(`swiglu_bwd`) ran on the backward's second stream" in open(md).read()
+
+
+# The layer's launch sequences. Routing: the fused kernel alone, after a count, after a
+# count and a scan, or (above 1024 experts) count, scan, scatter and both tile lists. Row
+# GEMMs: streaming or 256-row tiles, on the routing's lists or each on its own.
+FUSED = ["route_fused_kernel(int)"]
+COUNTED = ["route_count_kernel(int)", "route_fused_kernel(int)"]
+SCANNED = ["route_count_kernel(int)", "route_scan_kernel(int)", "route_fused_kernel(int)"]
+MANY = ["route_count_kernel(int)", "route_scan_kernel(int)", "route_scatter_wave_kernel(int)",
+        "build_tiles_kernel(int)", "build_tiles_kernel(int)"]
+STREAM = "void (anonymous namespace)::stream_rows_kernel<512, 32, 3, 1, 1, 0, 1>((anonymous namespace)::RowsArgs)"
+ROWS256 = "void (anonymous namespace)::grouped_rows_kernel<256, 256, 64, 2, 1, 0, 256, 0, true>(x)"
+
+
+def _sequence(routing, gemm, own_lists, backward):
+    one = (["build_tiles_kernel(int)"] if own_lists else []) + [gemm]
+    seq = [("route", n) for n in routing]
+    seq += [("fc1_swiglu", n) for n in one] + [("fc2", n) for n in one] + [("combine", "void combine_items_kernel<2, 8>(x)")]
+    if backward:
+        seq += [("fc2_dgrad", n) for n in one] + [("swiglu_bwd", "void swiglu_bwd_kernel<0, 0>(x)"),
+                                                  ("act_recompute", "void gated_act_kernel<0, 0>(x)"),
+                                                  ("fc2_wgrad", "void wgrad_persist_kernel<3>(x)")]
+        seq += [("fc1_dgrad", n) for n in one] + [("combine_bwd", "void combine_items_kernel<2, 8>(x)"),
+                                                  ("fc1_wgrad", "void wgrad_persist_kernel<3>(x)")]
+    return seq
+
+
+@pytest.mark.parametrize("routing", [FUSED, COUNTED, SCANNED, MANY], ids=["fused", "counted", "scanned", "many"])
+@pytest.mark.parametrize("gemm", [STREAM, ROWS256], ids=["stream", "rows256"])
+@pytest.mark.parametrize("own_lists", [False, True])
+@pytest.mark.parametrize("backward", [False, True])
+def test_launch_sequences(routing, gemm, own_lists, backward):
+    if own_lists and routing is MANY:
+        routing = MANY[:3]  # mm_route writes no lists
+    seq = _sequence(routing, gemm, own_lists, backward)
+    names = ["void at::native::fill(x)"] + ([n for _, n in seq] + ["void at::native::copy(x)"]) * 3
+    disp = [(i, n, 100 * i, 100 * i + 50, 0.0) for i, n in enumerate(names)]
+    steps = R.split_steps(disp)
+    assert len(steps) == 3
+    for step in steps:
+        want = {}
+        for stage, n in seq:
+            want.setdefault(stage, []).append(n)
+        assert {k: [d[1] for d in v] for k, v in R.assign_stages(step).items()} == want
