@@ -10,8 +10,8 @@
 // MI355X design: no global atomics, no host sync, no sort.
 // Up to 1024 experts (route_fused_kernel): a unit is 2048 consecutive routes
 // and one 16-wavefront workgroup. A workgroup needs, per expert, the routes in
-// earlier units and in all units; mostly it counts them itself from the ids
-// (L2-resident), so routing is ONE launch; else a first launch writes
+// earlier units and in all units; up to 32768 routes it counts them itself from
+// the ids (L2-resident), so routing is ONE launch; above, a first launch writes
 // unit_counts[unit][expert], and every workgroup sums the table or a second
 // launch scans it (see units_source). A block scan over the experts then
 // gives every expert's
@@ -22,8 +22,8 @@
 // M-tile lists of the row GEMMs.
 // It is latency-bound. Three launches (count, scan, scatter) without tile
 // lists measured, against this form with them (graph replay, us): 8 routes
-// over 128 experts 10.1 -> 5.9, 4084 over 60 17.0 -> 8.0, 32768 over 32 19.6
-// -> 11.2, 65536 over 896 27.2 -> 15.9; each tile list built by itself was
+// over 128 experts 10.3 -> 6.4, 4084 over 60 17.6 -> 8.7, 32768 over 32 19.4
+// -> 11.0, 65536 over 896 27.1 -> 17.7; each tile list built by itself was
 // another 3 to 7 us launch, two per forward and two per backward.
 // Above 1024 experts (up to 32768, bounded by LDS) count, scan and a
 // one-wavefront scatter per unit remain three launches (the reference's
@@ -150,7 +150,8 @@ __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
     int32_t* __restrict__ send_route, int32_t* __restrict__ send_token,
     int32_t* __restrict__ route_to_send, float* __restrict__ weight_perm, TileList* __restrict__ tlS,
     TileList* __restrict__ tl256) {
-  __shared__ int seg[kFusedWaves * kFusedExperts];  // [wave][expert]: routes of the segment, then its next row
+  // [wave][expert]: routes of the segment, then its next row
+  __shared__ __attribute__((aligned(16))) int seg[kFusedWaves * kFusedExperts];
   __shared__ int before[kFusedExperts], rest[kFusedExperts];  // routes in earlier / later units
   __shared__ uint64_t part[kFusedWaves];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
   for (int e = tid; e < E; e += kFusedThreads) before[e] = rest[e] = 0;
   __syncthreads();
 
-  // own unit: counts per wavefront segment (wave w owns routes start + w * kSeg ..)
+  // own unit: wave w owns routes start + w * kSeg ..
   constexpr int ITERS = kSeg / 64;
   int key[ITERS];
 #pragma unroll
@@ -170,17 +171,33 @@ __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
     const int64_t i = start + wave * kSeg + it * 64 + lane;
     const int e = i < R ? sel[i] : -1;
     key[it] = route_valid(e, E) ? e : E;
-    if (key[it] < E) atomicAdd(&seg[wave * E + key[it]], 1);
   }
   if (source == UNITS_SCANNED) {
     for (int e = tid; e < E; e += kFusedThreads) before[e] = unit_counts[static_cast<int64_t>(u) * E + e];
   } else if (source == UNITS_TABLE) {
-    for (int i = tid; i < nunits * E; i += kFusedThreads) {
-      const int v = i / E, e = i - v * E;
-      const int c = unit_counts[i];
-      if (v != u && c) atomicAdd(v < u ? &before[e] : &rest[e], c);
+    // thread (g, e) sums column e of every G-th row, 16 rows in flight
+    const int G = kFusedThreads / E, g = tid / E, e = tid - g * E;
+    if (g < G) {
+      int b = 0, r = 0;
+      for (int v = g; v < nunits; v += 16 * G) {
+        int c[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) c[j] = unit_counts[static_cast<int64_t>(min(v + j * G, nunits - 1)) * E + e];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int w = v + j * G;
+          b += w < u ? c[j] : 0;
+          r += w > u && w < nunits ? c[j] : 0;
+        }
+      }
+      atomicAdd(&before[e], b);
+      atomicAdd(&rest[e], r);
     }
-  } else {
+  } else if (nunits > 1) {
+    // Eight copies of each histogram (in seg, not yet in use), one per eight
+    // lanes: ids that repeat within a wavefront (a hot expert's) queue up on
+    // their LDS word.
+    const int copy = (lane >> 3) & 7;
     auto count = [&](int64_t lo, int64_t hi, int* hist) {
       int64_t i = lo + tid;
       for (; i + 7 * kFusedThreads < hi; i += 8 * kFusedThreads) {
@@ -189,16 +206,32 @@ __global__ __launch_bounds__(kFusedThreads) void route_fused_kernel(
         for (int j = 0; j < 8; ++j) e[j] = sel[i + j * kFusedThreads];
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-          if (route_valid(e[j], E)) atomicAdd(&hist[e[j]], 1);
+          if (route_valid(e[j], E)) atomicAdd(&hist[e[j] * 8 + copy], 1);
       }
       for (; i < hi; i += kFusedThreads) {
         const int e = sel[i];
-        if (route_valid(e, E)) atomicAdd(&hist[e], 1);
+        if (route_valid(e, E)) atomicAdd(&hist[e * 8 + copy], 1);
       }
     };
-    count(0, start, before);
-    count(end, R, rest);
+    static_assert(kFusedWaves == 16, "two histograms of eight copies fill seg");
+    count(0, start, seg);
+    count(end, R, seg + 8 * E);
+    __syncthreads();
+    if (tid < E) {
+      auto take = [](int* p) {  // sums a copy set and clears it
+        int4* q = reinterpret_cast<int4*>(p);
+        const int4 a = q[0], b = q[1];
+        q[0] = q[1] = make_int4(0, 0, 0, 0);
+        return a.x + a.y + a.z + a.w + b.x + b.y + b.z + b.w;
+      };
+      before[tid] = take(seg + tid * 8);
+      rest[tid] = take(seg + (E + tid) * 8);
+    }
+    __syncthreads();
   }
+#pragma unroll
+  for (int it = 0; it < ITERS; ++it)
+    if (key[it] < E) atomicAdd(&seg[wave * E + key[it]], 1);
   __syncthreads();
 
   // per expert: first row of every segment relative to the expert, then the
@@ -333,18 +366,19 @@ extern "C" size_t mm_route_workspace_bytes(int64_t num_routes, int32_t num_exper
 
 namespace {
 
-// Recounting costs each workgroup R ids, the table its R / 2048 * E entries
-// and a launch; measured (us, recount / table): 65536 routes 14.3 / 13.1 over
-// 128 experts and 15.9 / 23.9 over 896; 131072 routes over 32 experts 21.7 /
-// 12.8. At 32768 routes and below the launch alone costs more (11.2 over 32
-// experts, all of it). Both grow with the square of R, the scan does not: it
-// takes over at 2e8 ids or entries over all units (524288 routes over 600
-// experts, 1.3e8: 58 us recounted against 77 with a scan; 1048576 over 896,
-// 5.4e8: 191 against 153; 1048576 over 32, 8.4e6: 42 against 96).
+// Recounting costs each workgroup R ids and their LDS atomics, the table its
+// R / 2048 * E entries and a launch. Measured (us, recount / table): 32768
+// routes over 8 experts 10.6 / 11.6, over 896 13.3 / 14.5; 65536 over 8 14.2 /
+// 9.8, over 896 16.1 / 16.3. With every id the same the atomics of a histogram
+// queue up: 32768 routes 13.9 / 11.6 with the eight copies (one histogram: 33;
+// 524288 over 896 experts: 450, the table 36).
+// Reading the table grows with the square of R, the scan does not: it takes
+// over at 6e8 entries over all units (summed / scanned: 1048576 routes over
+// 1024 experts, 2.7e8, 134 / 159; 4194304 over 128, 5.4e8, 246 / 377; over
+// 512, 2.1e9, 790 / 507).
 int units_source(int64_t num_routes, int E, int64_t nunits) {
-  const bool recount = num_routes <= 32768 || E >= 512;
-  if (nunits * (recount ? num_routes : nunits * E) > 200000000) return UNITS_SCANNED;
-  return recount ? UNITS_RECOUNT : UNITS_TABLE;
+  if (num_routes <= 32768) return UNITS_RECOUNT;
+  return nunits * nunits * E > 600000000 ? UNITS_SCANNED : UNITS_TABLE;
 }
 
 int route_launch(const int32_t* selected, int64_t num_routes, int32_t top_k, int32_t num_experts,

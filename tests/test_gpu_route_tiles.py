@@ -1,6 +1,7 @@
 """Routing in one launch and the M-tile lists it writes (GPU): units of 2048
-routes, the switch above 32768 routes and below 512 experts from recounting
-in every workgroup to a count table, from both to a scanned table, and the switch at 1024 experts to the large-expert kernels."""
+routes, the switch above 32768 routes from recounting in every workgroup to a
+count table, from that to a scanned table, and the switch at 1024 experts to
+the large-expert kernels."""
 
 import numpy as np
 import pytest
@@ -19,13 +20,20 @@ CASES = [
     (2048, 1, 1024, False),
     (2049, 1, 1023, True),
     (4096, 8, 32, False),    # 32768 routes: the last recounting size
+    (16384, 2, 8, True),     # the same, repeated ids in every wavefront
+    (2049, 1, 1, True),
     (32769, 1, 33, False),   # the first size with a count table
     (32769, 1, 511, False),
-    (32769, 1, 512, False),  # recounting again
+    (32769, 1, 512, False),
+    (32769, 1, 1, True),     # 1024 rows of the table at a time, 17 units
+    (34817, 1, 1000, True),
     (8192, 16, 896, False),
-    (39900, 16, 600, False),   # 312 units: recounted; the next one is scanned
+    (39900, 16, 600, False),
     (41000, 16, 600, False),
-    (83000, 16, 500, True),    # 649 units: scanned instead of summed
+    (83000, 16, 500, True),
+    (120000, 16, 600, False),  # 938 units: summed; the next ones are scanned
+    (131073, 16, 600, False),
+    (131073, 16, 600, True),
     (300, 3, 1025, False),
 ]
 
