@@ -12,7 +12,8 @@
 //    v_mfma_f32_32x32x16_bf16, each wave owning a (BM / WM) x (BN / WN)
 //    sub-tile. 256 x 256 tiles with K >= 1024 run 4 wavefronts of 128 x 128
 //    (one per SIMD, accumulators in the AGPRs) with register-staged operand
-//    copies interleaved with the MFMAs. Experts averaging fewer than 148 rows
+//    copies interleaved with the MFMAs; where N is no multiple of 256 the
+//    tiles are 256 x 128. Experts averaging fewer than 148 rows (160 there)
 //    run weight-streaming tiles of at most 160 rows, split by columns only.
 //  * Otherwise operands go global -> LDS with gfx950 LDS-DMA
 //    (global_load_lds_dwordx4) through an NST-stage ring, one barrier per K
@@ -1646,16 +1647,24 @@ int device_cus() {
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Row-GEMM tile height: weight-streaming tiles of at most 160 rows while
-// experts average fewer than 148 rows (or N is no multiple of 256), 256 x 256
-// tiles above. Either way an expert's weights should be read once, so the
-// streaming tile must hold most experts: 160 rows hold an average of 128 with
-// softmax top-k routing, and past 148 half the experts would need a second
-// tile. Measured, us streaming / 256 x 256, 128 experts: FC1 of 7168 x 4096
-// at 96 rows 1195 / 1419, 128 rows 1363 / 1580, 146 rows 1554 / 1699; FC2 of
-// 2048 x 7168 624 / 784, 700 / 882, 791 / 932; 2048 x 1536 at 140 rows 192 /
-// 201, 150 rows 212 / 208, 170 rows 284 / 207.
+// experts average fewer than 148 rows (160 where N is no multiple of 256),
+// tiles of 256 rows by 256 (128) columns above. Either way an expert's weights
+// should be read once, so the streaming tile must hold most experts: 160 rows
+// hold an average of 128 with softmax top-k routing, and past 148 half the
+// experts would need a second tile. Measured, us streaming / 256 x 256, 128
+// experts: FC1 of 7168 x 4096 at 96 rows 1195 / 1419, 128 rows 1363 / 1580,
+// 146 rows 1554 / 1699; FC2 of 2048 x 7168 624 / 784, 700 / 882, 791 / 932;
+// 2048 x 1536 at 140 rows 192 / 201, 150 rows 212 / 208, 170 rows 284 / 207.
+// Streaming / 256 x 128, FC2 input gradient of 60 experts of 2304 x 896: 150
+// rows 77 / 81, 160 rows 100 / 85, 600 rows 255 / 217, 2000 rows 800 / 579
+// (tiles of 128 x 128 in 4 waves: 99, 104, 246, 685).
+// The average also stands for skewed routing, where most rows lie in a few
+// experts of many tiles. With Zipf 1.2 over 64 experts of 4096 x 1536, us
+// streaming / the 256-row tiles from an average of 96 on: 100 rows FC1 400 /
+// 402, FC2 182 / 220, FC2 input gradient 214 / 197, FC1 input gradient 373 /
+// 432; 140 rows 442 / 432, 207 / 242, 249 / 210, 420 / 454.
 int pick_rows_bm(int64_t max_rows, int E, int n) {
-  return n % 256 == 0 && max_rows >= 148 * static_cast<int64_t>(E) ? 256 : kStreamRows;
+  return max_rows >= (n % 256 == 0 ? 148 : 160) * static_cast<int64_t>(E) ? 256 : kStreamRows;
 }
 
 template <class Launch>
@@ -1809,7 +1818,9 @@ int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const 
     if (int rc = mm_build_tiles(offsets, E, bm, static_cast<TileList*>(ts.workspace), s)) return rc;
     p.tl = static_cast<const TileList*>(ts.workspace);
   }
-  if (bm == 256) {
+  if (bm == 256 && p.n % 256 != 0) {
+    launch_rows_cfg<256, 128, 64, 3, BLAYOUT, EPI, 512>(p, max_rows, E, s);
+  } else if (bm == 256) {
     if (rows_lds_dma() || p.k < 1024)
       launch_rows_cfg<256, 256, 64, 2, BLAYOUT, EPI, 512>(p, max_rows, E, s);
     else

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 # multiple of 512) 512-column tiles, and 256 x 256 tiles (148 rows on average)
 @pytest.mark.parametrize("k", [64, 320, 1088])  # 1088: the register-staged 256 x 256 tiles
 @pytest.mark.parametrize("n_contig", [True, False])
-@pytest.mark.parametrize("n", [512, 768])
+@pytest.mark.parametrize("n", [384, 512, 768])
 def test_row_gemm(k, n_contig, n):
     from mega_moe.ops import _kernels as K
 
