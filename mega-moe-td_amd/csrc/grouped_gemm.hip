@@ -1401,11 +1401,16 @@ struct TileCursor {
 // that expert's per_e tiles) and an even share of the rest. Each wave finds
 // the same answer from the offsets before its first copy (lane l sums experts
 // l, l + 64, ..., which are all of team l % nteams).
+// (16 experts of 16 x 8 tiles, 256 workgroups, us at 256 / 512 / 1024 rows:
+// 113 / 190 / 345, i.e. 1.2 us for each step of a tile and 4 steps besides;
+// below 256 rows the stores alone are the time, 80 us.)
 // One team shares any split of the rows, but reads each expert's rows into
-// every XCD's L2. Measured, dW1, teams -> one team: even experts slower (100
-// of 8 x 6 tiles: 157 -> 165 us), Zipf-routed ones faster where the busiest
-// team has many tiles (64 of 16 x 12 tiles: 1286 -> 501 us) but not where the
-// longest expert's single round is the time (256 of 4 x 4: 329 -> 359 us).
+// every XCD's L2. Measured, us, teams / one team / this rule: top-k routing,
+// 140 rows on average, 128 experts of 8 x 6 tiles 224 / 236 / 219, 60 of 9 x 7
+// 158 / 159 / 146; Zipf routing 64 experts of 16 x 12 tiles 701 / 477 / 466,
+// 128 of 8 x 6 358 / 275 / 273, 256 of 16 x 8 2169 / 1337 / 1308, but where the
+// longest expert's single round is the time 256 of 4 x 4 246 / 274 / 249. It
+// misses some short rounds: 60 of 9 x 3 at 64 rows 83 / 64 / 82.
 constexpr int kTileStoreSteps = 4;
 __device__ __forceinline__ bool teams_uneven(const int32_t* offsets, int E, int rows_cap, int nteams, int nc,
                                              int per_e) {
@@ -1450,14 +1455,19 @@ __global__ __launch_bounds__(512) void wgrad_persist_kernel(WgradArgs a, int num
   // walking its own experts: team q of XCD x0 takes experts x0 + 8q,
   // x0 + 8q + 8 * teams, ... (16 workgroups per expert measured 2% faster
   // than 32 on the Kimi-scale gradients, and 4 teams no faster than 2). With
-  // fewer experts than teams, or rows that load the teams unevenly, the whole
-  // grid is one team, if that gives every workgroup tiles to walk.
+  // fewer experts than teams the whole grid is one team as soon as that gives
+  // every workgroup a tile (us, teams / one team: one expert of 256 tiles and
+  // 140 rows 126 / 15, 4 of 64 34 / 15, 8 of 64 36 / 26, 14 of 36 31 / 26, 15
+  // of 32 24.2 / 25.2), with more where its rows load the teams unevenly.
   const int per_xcd = gridDim.x / kXcds;
   const int teams = per_xcd % 2 == 0 ? 2 : 1;
   const int team = (blockIdx.x / kXcds) % teams;
-  const bool one_team = num_experts * (a.n1 / BM) * (a.n2 / BN) > 2 * static_cast<int>(gridDim.x) &&
-                        (num_experts < kXcds * teams || teams_uneven(a.offsets, num_experts, a.rows_cap, kXcds * teams, per_xcd / teams,
-                                      (a.n1 / BM) * (a.n2 / BN)));
+  const int tiles = num_experts * (a.n1 / BM) * (a.n2 / BN);
+  const bool one_team =
+      num_experts < kXcds * teams
+          ? tiles >= static_cast<int>(gridDim.x)
+          : tiles > 2 * static_cast<int>(gridDim.x) &&
+                teams_uneven(a.offsets, num_experts, a.rows_cap, kXcds * teams, per_xcd / teams, (a.n1 / BM) * (a.n2 / BN));
   const int x = one_team ? 0 : blockIdx.x % kXcds + team * kXcds;
   const int c = one_team ? blockIdx.x : blockIdx.x / kXcds / teams;
   const int nc = one_team ? gridDim.x : per_xcd / teams;
