@@ -144,6 +144,17 @@ int mm_permute(const uint16_t* x, int64_t ldx, const int32_t* send_token,
 size_t mm_gemm_workspace_bytes(int64_t max_rows, int32_t num_experts);
 
 /*
+ * Rows and columns of the tiles that mm_grouped_gemm of these sizes runs on
+ * the current device (n_contiguous: b_sn == 1); for mm_fc1_swiglu n = 2 *
+ * inter, k = hidden, n_contiguous = 1, saves_fc1 = (fc1_out != NULL). A
+ * 160-row tile holds up to 160 rows of one expert. The choice does not change
+ * a result: every tile sums an element's products over ascending k.
+ */
+int mm_row_tile(int64_t max_rows, int32_t num_experts, int32_t n, int32_t k,
+                int32_t n_contiguous, int32_t saves_fc1, int32_t* rows,
+                int32_t* columns);
+
+/*
  * FC1 grouped GEMM with the gated activation fused into its epilogue.
  * Replaces kernels/dispatch_fc1.py:580-752 + kernels/weighted_swiglu.py:18-81
  * and the FC1 leg of kernels/fused_forward.py:551-1008.

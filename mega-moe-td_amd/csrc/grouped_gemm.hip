@@ -1752,8 +1752,14 @@ bool rows_lds_dma() {
 // share (112 experts of 2048 x 1536: 111 against 124 us), unless all weights
 // the call touches are small enough to be found in the 256 MiB memory-side
 // cache by the next call (8 experts, 50 MB: 17 us against 21; 16 experts, 67
-// MB: 17 against 19; 134 MB: 38 against 35).
-// MM_WEIGHT_NT=0 drops the hint (read on every call).
+// MB: 17 against 19; 134 MB: 38 against 35). That next call must want the same
+// weights: one layer again, or its backward. Where a pass over many layers
+// lies between, the hint would be the better choice (forward of one token, 8
+// experts of 2048 x 768, us without / with it: weights repeated 30.1 / 32.9,
+// rotated through 1.2 GB 36.5 / 34.2; of two tokens 37.4 / 38.6 and 43.4 /
+// 39.5), and the call cannot know.
+// MM_WEIGHT_NT=0 drops the hint (read on every call) from tiles of 128 and 256
+// columns; 512 columns are read with it in any case.
 struct StreamCfg {
   int bn;
   bool nt;
@@ -1804,6 +1810,18 @@ bool wgrad_reg(int64_t max_rows, int E) {
 }
 bool wgrad_small_k(int64_t max_rows, int E) { return max_rows <= kSmallKRows * static_cast<int64_t>(E); }
 
+// Rows and columns of the tiles of a row GEMM, and (streaming tiles) the hint.
+struct RowTile {
+  int bm;
+  StreamCfg cfg;
+};
+
+RowTile pick_row_tile(int64_t max_rows, int E, int n, int k, bool n_contig, bool save) {
+  const int bm = pick_rows_bm(max_rows, E, n);
+  if (bm == kStreamRows) return {bm, pick_stream_cfg(max_rows, E, n, k, n_contig, save)};
+  return {bm, {n % 256 == 0 ? 256 : 128, false}};
+}
+
 // The M-tile list of a row GEMM: the lists mm_route_tiles wrote (lists), or
 // one made here from offsets (workspace).
 struct TileSource {
@@ -1815,7 +1833,7 @@ struct TileSource {
 template <int BLAYOUT, int EPI>
 int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const TileSource& ts, hipStream_t s,
              const char* what) {
-  const int bm = pick_rows_bm(max_rows, E, p.n);
+  const auto [bm, c] = pick_row_tile(max_rows, E, p.n, p.k, BLAYOUT == B_NCONTIG, p.fc1_out != nullptr);
   // the largest grid any tile configuration launches (the shortest M tiles
   // padded to a multiple of 8, 128-wide N tiles) must fit a 32-bit grid size
   if ((mm_max_m_tiles(max_rows, E, kStreamRows) + kXcds - 1) / kXcds * kXcds * (p.n / 128) >= (int64_t(1) << 31)) {
@@ -1828,7 +1846,7 @@ int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const 
     if (int rc = mm_build_tiles(offsets, E, bm, static_cast<TileList*>(ts.workspace), s)) return rc;
     p.tl = static_cast<const TileList*>(ts.workspace);
   }
-  if (bm == 256 && p.n % 256 != 0) {
+  if (bm == 256 && c.bn == 128) {
     launch_rows_cfg<256, 128, 64, 3, BLAYOUT, EPI, 512>(p, max_rows, E, s);
   } else if (bm == 256) {
     if (rows_lds_dma() || p.k < 1024)
@@ -1836,7 +1854,6 @@ int run_rows(RowsArgs p, const int32_t* offsets, int64_t max_rows, int E, const 
     else
       launch_rows_cfg<256, 256, 64, 2, BLAYOUT, EPI, 256, true>(p, max_rows, E, s);
   } else {
-    const StreamCfg c = pick_stream_cfg(max_rows, E, p.n, p.k, BLAYOUT == B_NCONTIG, p.fc1_out != nullptr);
     if constexpr (BLAYOUT == B_NCONTIG) {
       if (c.bn == 512) {
         launch_stream<512, 32, 3, BLAYOUT, EPI, 1>(p, max_rows, E, s);
@@ -1985,6 +2002,16 @@ extern "C" int mm_grouped_gemm_tiles(const uint16_t* a, int64_t lda, const int32
   MM_CHECK_ARG(tiles, "mm_grouped_gemm_tiles: null pointer");
   return grouped_gemm(a, lda, a_rows, b, b_se, b_sn, b_sk, offsets, num_experts, max_rows, n, k, c, ldc,
                       TileSource{tiles, nullptr, tiles_bytes}, stream, "mm_grouped_gemm_tiles");
+}
+
+extern "C" int mm_row_tile(int64_t max_rows, int32_t num_experts, int32_t n, int32_t k, int32_t n_contiguous,
+                           int32_t saves_fc1, int32_t* rows, int32_t* columns) {
+  MM_CHECK_ARG(max_rows >= 0 && num_experts > 0 && n > 0 && n % 128 == 0 && k > 0 && rows && columns,
+               "mm_row_tile: bad sizes");
+  const RowTile t = pick_row_tile(max_rows, num_experts, n, k, n_contiguous != 0, saves_fc1 != 0);
+  *rows = t.bm;
+  *columns = t.cfg.bn;
+  return MM_OK;
 }
 
 extern "C" size_t mm_gemm_workspace_bytes(int64_t max_rows, int32_t num_experts) {

@@ -48,6 +48,7 @@ SIGNATURES = {
                                            _F32, _F32, _F32, _P, _P, _I32, _P, _P, _SZ, _P]),
     "mm_grouped_gemm_tiles": (ctypes.c_int, [_P, _I64, _P, _P, _I64, _I64, _I64, _P, _I32, _I64, _I32,
                                              _I32, _P, _I64, _P, _SZ, _P]),
+    "mm_row_tile": (ctypes.c_int, [_I64, _I32, _I32, _I32, _I32, _I32, _P, _P]),
     "mm_grouped_wgrad": (ctypes.c_int, [_P, _I64, _P, _P, _I64, _P, _P, _I32, _I64, _I32, _I32, _P, _P,
                                         _SZ, _P]),
     "mm_combine": (ctypes.c_int, [_P, _I64, _P, _I64, _I32, _I32, _P, _I64, _P]),

@@ -75,3 +75,26 @@ def test_grouped_gemm_rejects_grids_past_32_bits():
     max_rows, E, n, k = (1 << 31) - 1, 8, 65536, 64
     rc = lib.mm_grouped_gemm(fake, k, None, fake, n * k, 1, n, fake, E, max_rows, n, k, fake, n, fake, 1 << 40, None)
     assert rc == -1 and b"too many tiles" in lib.mm_last_error()
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.library_path()), reason="libmegamoe.so not built")
+@pytest.mark.parametrize("max_rows,E,n,n_contig,saves,tile", [
+    (8, 128, 1536, 1, 0, (160, 128)), (8, 128, 1536, 1, 1, (160, 256)),   # one token: one round of 128 columns
+    (65536, 896, 4096, 1, 1, (160, 512)), (65536, 896, 7168, 0, 0, (160, 256)),
+    (147, 1, 1024, 1, 0, (160, 128)), (148, 1, 1024, 1, 0, (256, 256)),   # the line between tile heights
+    (159, 1, 896, 0, 0, (160, 128)), (160, 1, 896, 0, 0, (256, 128)),     # N no multiple of 256
+])
+def test_row_tile(max_rows, E, n, n_contig, saves, tile):
+    lib = _lib.load()
+    rows, cols = ctypes.c_int32(), ctypes.c_int32()
+    assert lib.mm_row_tile(max_rows, E, n, 1024, n_contig, saves, ctypes.byref(rows), ctypes.byref(cols)) == 0
+    assert (rows.value, cols.value) == tile
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.library_path()), reason="libmegamoe.so not built")
+def test_row_tile_rejects_bad_sizes():
+    lib = _lib.load()
+    out = ctypes.c_int32()
+    for args in ((-1, 1, 128, 64), (1, 0, 128, 64), (1, 1, 100, 64), (1, 1, 128, 0)):
+        assert lib.mm_row_tile(*args, 1, 0, ctypes.byref(out), ctypes.byref(out)) == -1
+    assert lib.mm_row_tile(1, 1, 128, 64, 1, 0, None, ctypes.byref(out)) == -1

@@ -164,10 +164,11 @@ def test_grouped_gemm_ragged_tails(layout, gather):
 
 
 @pytest.mark.parametrize("layout", ["kcontig", "ncontig"])
-@pytest.mark.parametrize("E,N", [(13, 512), (37, 256)])
+@pytest.mark.parametrize("E,N", [(13, 512), (37, 256), (67, 256), (101, 512)])
 def test_weight_streaming_xcd_mapping(layout, E, N, monkeypatch):
-    """128-row tiles (experts averaging under 96 rows) run M tile m on XCD
-    m % 8; with a tile count that is no multiple of 8 (surplus workgroups
+    """Weight-streaming tiles (experts averaging under 148 rows) run M tile m
+    on XCD m % 8, or, where the bound of M tiles is below 64 (E = 13, 37), in
+    flat order; with a tile count that is no multiple of 8 (surplus workgroups
     exit) the result is bit-identical to the contiguous per-XCD split
     (MM_XCD_MOD=0) and matches the fp32 reference."""
     from mega_moe.ops import _kernels as K
@@ -175,6 +176,7 @@ def test_weight_streaming_xcd_mapping(layout, E, N, monkeypatch):
     counts = torch.randint(0, 140, (E,), generator=g0).tolist()
     offs = torch.tensor([0] + list(np.cumsum(counts)), dtype=torch.int32, device=DEV)
     M, Kd = int(offs[-1]), 320
+    assert (M // 160 + E >= 64) == (E >= 64) and sum(c > 0 for c in counts) % 8
     g = torch.Generator(device=DEV).manual_seed(7)
     a = torch.randn(M + 5, Kd, device=DEV, generator=g).to(torch.bfloat16)
     a_rows = torch.randperm(M + 5, device=DEV, generator=g)[:M].to(torch.int32)

@@ -188,10 +188,10 @@ def test_full_size_sampled_parity(name, fmt, activation):
     against the CPU oracle, max relative error <= 2e-2 plus the reference's
     GRAD element check. (E32 is a forward-only config; its backward is
     checked too.) The Kimi layer also runs with the FP8 FC1 save, the
-    backward reading the E4M3 values and scales (128-row tiles), the
+    backward reading the E4M3 values and scales (streaming tiles), the
     Qwen-like layer with the SiTU-GLU and clamped SwiGLU activations and the
     FP8 save (256-row register-staged tiles), and the DeepSeek-V3-like layer
-    (256 experts averaging 128 rows, 256-row tiles)."""
+    (256 experts averaging 128 rows, streaming tiles of up to 160)."""
     spec = CASES[name]
     inp = make_inputs(spec, device="cuda", seed=1234)
     kw = _act_kw(activation)
