@@ -130,9 +130,11 @@ class FusedMoEForward(torch.nn.Module):
         # (MOE_FWD_TIMING=1 attaches one, as the reference's phase stamps are
         # switched on by that variable, ops/forward.py:1656-1660)
         self.stage_timer = StageTimer() if os.environ.get("MOE_FWD_TIMING", "0") == "1" else None
-        # operator-owned workspaces (routing scratch, tile lists, weight-gradient
-        # operand staging), sized for max_tokens_per_rank at the first forward so
-        # that they never move afterwards (a captured graph keeps their addresses)
+        # operator-owned workspaces of the calls issued one entry point at a time
+        # (routing plans, staged passes, a backward without tile lists), sized for
+        # max_tokens_per_rank at the first routing so that they never move
+        # afterwards (a captured graph keeps their addresses); the one-call
+        # forward and backward bring their own scratch
         self._workspaces = K.WorkspacePool()
         self._ws_ready = False
 
@@ -424,7 +426,6 @@ class FusedMoEForward(torch.nn.Module):
                 return out
         tables = None
         if num_tokens and self.stage_timer is None:
-            self._reserve_workspaces(hidden_states.device)
             if return_saved:
                 tables = RouteTables(num_routes, self.experts_per_rank, self.top_k, hidden_states.device, True, True)
             out, act, fc1_out, fc1_scale = K.layer_forward(

@@ -89,3 +89,16 @@ def test_replaced_offsets_are_read():
         got.append(mega_moe.moe_backward_triton(saved, inp["dy"]))
     for k in GRADS:
         assert torch.equal(got[0][k], got[1][k]), k
+
+
+def test_one_call_holds_no_workspaces():
+    spec = CaseSpec("held", 64, 256, 128, 4, 2, "softmax_topk", True)
+    inp = make_inputs(spec, device="cuda", seed=6, weight_scale=0.1)
+    op = _op(spec, "bf16")
+    args = (inp["x"], inp["selected"], inp["gate_up"], inp["down"], inp["rw"])
+    op.forward(*args)
+    _, saved = op.forward(*args, return_saved=True)
+    mega_moe.moe_backward_triton(saved, inp["dy"])
+    assert op._workspaces.nbytes() == 0  # the passes bring their own scratch
+    op.build_routing_plan(inp["selected"])
+    assert op._workspaces.nbytes() > 0
