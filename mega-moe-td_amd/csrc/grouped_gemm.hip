@@ -1146,13 +1146,18 @@ __device__ __attribute__((aligned(256))) bf16 g_wgrad_zero_row[256];  // never w
 // Wave w copies the stage's K rows 16w .. 16w + 15 (two per 1 KiB chunk);
 // the row ids of a gathered operand arrive one stage earlier, one load per
 // wave (lanes 0..15), and are broadcast with readlane. Rows of both operands
-// past the expert's end are read from a zero row, so the loop body has no
-// branch: the row there may be another expert's or, past the last expert of
-// a call with dropped routes, one that was never written, and a zero times an
-// infinity or a NaN is a NaN. The
+// past the expert's end count as zeros, without a branch in the loop: the row
+// there may be another expert's or, past the last expert of a call with
+// dropped routes, one that was never written, and a zero times an infinity or
+// a NaN is a NaN. P rows there come from a zero row; Q rows, where Q isn't
+// gathered and an expert's rows fit 32-bit offsets (QBUF), through a buffer
+// descriptor that ends with the expert's last row, which also spares the
+// 64-bit address arithmetic (us, zero row for P alone / for both / descriptor
+// for Q: 32 experts of 4096 rows, 4096 x 3072 3130 / 3220 / 3083; 16 of 4000,
+// 6400 x 2048 1640 / 1678 / 1613), else from the zero row too. The
 // epilogue stages the tile in the (then idle) ring, XOR-swizzled, and stores
 // 2 rows x 512 B per instruction.
-template <int NT = 256>
+template <bool QBUF, int NT = 256>
 __global__ __launch_bounds__(NT) void wgrad_reg_kernel(WgradArgs a, int num_experts, int per_xcd) {
   constexpr int BM = 256, BN = 256, BK_ = 64, WN = 2, WM = NT / 64 / WN;
   using Mma = MmaTile<BM, BN, WM, WN>;
@@ -1191,6 +1196,11 @@ __global__ __launch_bounds__(NT) void wgrad_reg_kernel(WgradArgs a, int num_expe
     const int r = min(r0 + s * BK_ + wave * RPW + (lane & (RPW - 1)), cap1);
     return *(rows ? rows + r : a.offsets);
   };
+  // The zero row's address is read once: the compiler loads it through the GOT,
+  // with its wait, at every stage (12% of the time with QBUF; without it that
+  // schedule is the better one).
+  uint64_t zrow = reinterpret_cast<uint64_t>(g_wgrad_zero_row);
+  if constexpr (QBUF) asm volatile("" : "+s"(zrow));
   auto src = [&](const bf16* base, int64_t ld, const int32_t* rows, int ids, int s, int v, int64_t col0) {
     const int kl = wave * RPW + v * KPC + half;  // K row within the stage
     const int kg = r0 + s * BK_ + kl;            // row of the expert-major order
@@ -1198,19 +1208,37 @@ __global__ __launch_bounds__(NT) void wgrad_reg_kernel(WgradArgs a, int num_expe
     const int row = rows ? (half ? hi : lo) : min(kg, cap1);
     const int c = (lcol ^ mn_swz<16>(kl)) * 8;
     const uint64_t data = reinterpret_cast<uint64_t>(base + static_cast<int64_t>(row) * ld + col0 + c);
-    const uint64_t zero = reinterpret_cast<uint64_t>(g_wgrad_zero_row + c);
+    const uint64_t zero = zrow + 2 * c;
     const uint64_t addr = kg >= r1 ? zero : data;
     return *reinterpret_cast<const u32x4_t*>(addr);
   };
+  // QBUF: the descriptor covers the block's columns of the expert's rows; a
+  // 16-byte load at or past its end returns zeros (the host checks that an
+  // offset fits 32 bits and that a row is at least n2 long)
+  const uint32_t q_bytes =
+      r1 > r0 ? static_cast<uint32_t>(r1 - r0 - 1) * static_cast<uint32_t>(a.ldq * 2) + BN * 2 : 0;
+  const __amdgpu_buffer_rsrc_t q_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16*>(a.q + static_cast<int64_t>(r0) * a.ldq + qc), 0, q_bytes, 0x00020000);
+  auto src_q = [&](int s, int v) -> u32x4_t {
+    const int kl = wave * RPW + v * KPC + half;
+    const uint32_t at = static_cast<uint32_t>(s * BK_ + kl) * static_cast<uint32_t>(a.ldq * 2);
+    return __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, at + (lcol ^ mn_swz<16>(kl)) * 16, 0, 0);
+  };
   u32x4_t ra[PW], rb[PW];
-  int pid_cur = 0, qid_cur = 0, pid_nxt = 0, qid_nxt = 0;
+  int pid_cur = 0, pid_nxt = 0;
+  [[maybe_unused]] int qid_cur = 0, qid_nxt = 0;
   auto gload_p = [&](int s) {
 #pragma unroll
     for (int v = 0; v < PW; ++v) ra[v] = src(a.p, a.ldp, a.p_rows, pid_cur, s, v, pc);
   };
   auto gload_q = [&](int s) {
 #pragma unroll
-    for (int v = 0; v < PW; ++v) rb[v] = src(a.q, a.ldq, a.q_rows, qid_cur, s, v, qc);
+    for (int v = 0; v < PW; ++v) {
+      if constexpr (QBUF)
+        rb[v] = src_q(s, v);
+      else
+        rb[v] = src(a.q, a.ldq, a.q_rows, qid_cur, s, v, qc);
+    }
   };
   // chunk v of wave w sits at LDS chunk w * PW + v (rows 2 (w PW + v) + 0/1)
   auto put = [&](bf16* buf, const u32x4_t (&r)[PW]) {
@@ -1224,19 +1252,19 @@ __global__ __launch_bounds__(NT) void wgrad_reg_kernel(WgradArgs a, int num_expe
   Frag fa[2][Mma::MI], fb[2][Mma::NI];
   if (nk > 0) {
     pid_cur = load_ids(a.p_rows, 0);
-    qid_cur = load_ids(a.q_rows, 0);
+    if constexpr (!QBUF) qid_cur = load_ids(a.q_rows, 0);
     gload_p(0);
     gload_q(0);
     put(smem, ra);
     put(smem + PTile::ELEMS, rb);
     if (nk > 1) {
       pid_cur = load_ids(a.p_rows, 1);
-      qid_cur = load_ids(a.q_rows, 1);
+      if constexpr (!QBUF) qid_cur = load_ids(a.q_rows, 1);
       gload_p(1);
       gload_q(1);
       if (nk > 2) {
         pid_nxt = load_ids(a.p_rows, 2);
-        qid_nxt = load_ids(a.q_rows, 2);
+        if constexpr (!QBUF) qid_nxt = load_ids(a.q_rows, 2);
       }
     }
   }
@@ -1271,7 +1299,7 @@ __global__ __launch_bounds__(NT) void wgrad_reg_kernel(WgradArgs a, int num_expe
           put(nxt + PTile::ELEMS, rb);
           gload_q(s2);
           pid_nxt = load_ids(a.p_rows, min(kt + 3, nk - 1));
-          qid_nxt = load_ids(a.q_rows, min(kt + 3, nk - 1));
+          if constexpr (!QBUF) qid_nxt = load_ids(a.q_rows, min(kt + 3, nk - 1));
         }
 #pragma unroll
         for (int q = 0; q < Mma::MI * Mma::NI; ++q) {
@@ -2076,7 +2104,12 @@ extern "C" int mm_grouped_wgrad(const uint16_t* p, int64_t ldp, const int32_t* p
     grouped_wgrad_kernel<128, 128, 32, 2, true><<<grid, kThreads, 0, s>>>(a, num_experts, px);
   } else if (bm == 256 && bn == 256) {
     if (wgrad_reg(max_rows, num_experts)) {
-      wgrad_reg_kernel<><<<grid, 256, 0, s>>>(a, num_experts, px);
+      // offsets reach 63 rows past an expert's end
+      const bool qbuf = !q_rows && ldq >= n2 && max_rows + 64 < (int64_t(1) << 31) / ldq;
+      if (qbuf)
+        wgrad_reg_kernel<true><<<grid, 256, 0, s>>>(a, num_experts, px);
+      else
+        wgrad_reg_kernel<false><<<grid, 256, 0, s>>>(a, num_experts, px);
     } else {
       grouped_wgrad_kernel<256, 256, 64, 2, false, 512><<<grid, 512, 0, s>>>(a, num_experts, px);
     }

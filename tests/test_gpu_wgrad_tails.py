@@ -8,12 +8,13 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-# rows per expert choose the kernel: persistent, 64-row K steps, register-staged
+# rows per expert choose the kernel: persistent, 64-row K steps, register-staged (with
+# Q read through a buffer descriptor, or gathered by address)
 @pytest.mark.parametrize("counts,n1,n2", [
     ([70, 1, 33, 50], 512, 256), ([500, 333, 1, 800], 256, 512), ([500, 333], 128, 384),
-    ([2100, 2049, 2177, 2500], 256, 512),
+    ([2100, 2049, 2177, 2500], 256, 512), ([2112, 9000, 1, 0, 64, 4099], 512, 256),
 ])
-@pytest.mark.parametrize("gather", [False, True])
+@pytest.mark.parametrize("gather", ["none", "p", "pq"])
 def test_rows_past_the_end(counts, n1, n2, gather):
     from mega_moe.ops import _kernels as K
 
@@ -23,18 +24,20 @@ def test_rows_past_the_end(counts, n1, n2, gather):
     n, cap = int(offs[-1]), int(offs[-1]) + 100  # 100 capacity rows hold no route
     p = torch.randn(cap, n1, generator=g, device="cuda").bfloat16()
     q = torch.randn(cap, n2, generator=g, device="cuda").bfloat16()
-    rows = torch.randperm(cap, generator=g, device="cuda").int() if gather else None
-    prow = rows.long() if gather else torch.arange(cap, device="cuda")
+    straight = torch.arange(cap, device="cuda").int()
+    prow = torch.randperm(cap, generator=g, device="cuda").int() if "p" in gather else straight
+    qrow = torch.randperm(cap, generator=g, device="cuda").int() if "q" in gather else straight
     for bad, lo, hi in ((float("nan"), n, cap), (float("inf"), int(offs[1]), int(offs[2]))):
-        p[prow[lo:hi]] = bad  # never-written rows; all of expert 1
-        q[lo:hi] = bad
-    c = K.grouped_wgrad(p, rows, q, None, offs.cuda(), n1, n2, max_rows=cap)
+        p[prow[lo:hi].long()] = bad  # never-written rows; all of expert 1
+        q[qrow[lo:hi].long()] = bad
+    c = K.grouped_wgrad(p, prow if "p" in gather else None, q, qrow if "q" in gather else None, offs.cuda(), n1, n2,
+                        max_rows=cap)
     torch.cuda.synchronize()
     for e in range(E):
         r0, r1 = int(offs[e]), int(offs[e + 1])
         if e == 1:
             continue
-        pe, qe = p[prow[r0:r1]].float(), q[r0:r1].float()
+        pe, qe = p[prow[r0:r1].long()].float(), q[qrow[r0:r1].long()].float()
         ref, mag = pe.t() @ qe, pe.abs().t() @ qe.abs()
         err = (c[e].float() - ref).abs()
         # fp32 sums in two orders, one bf16 rounding
