@@ -226,7 +226,10 @@ struct KcTile {
 // cv ^ mn_swz(k). KD is the K depth of the MFMA that reads the fragments.
 // 16 (32x32x16): a 32-lane pass takes 64 bytes of 4 K rows. 32 (16x16x32): it
 // takes 32 bytes of 8 K rows (0-3 and 8-11, then 16-19 and 24-27). Either
-// way the pieces of a pass sit in distinct banks.
+// way the pieces of a pass taken like that sit in distinct banks. Counted
+// (SQ_LDS_BANK_CONFLICT / SQ_LDS_IDX_ACTIVE, Kimi-scale layer): 0.37 for the
+// 512-column streaming tiles and 0.29 for the small-K weight gradient, both
+// bound by HBM, against 0.01 for the K-contiguous streaming tiles.
 template <int KD>
 __device__ __forceinline__ int mn_swz(int k) {
   if constexpr (KD == 32)

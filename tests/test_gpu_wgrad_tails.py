@@ -42,3 +42,30 @@ def test_rows_past_the_end(counts, n1, n2, gather):
         err = (c[e].float() - ref).abs()
         # fp32 sums in two orders, one bf16 rounding
         assert bool((err <= 2.0 ** -8 * ref.abs() + (r1 - r0) * 2.0 ** -23 * mag).all()), (e, counts[e])
+
+
+@pytest.mark.parametrize("tokens,experts,top_k", [(60, 4, 2), (3000, 8, 2), (4700, 2, 1)])
+@pytest.mark.parametrize("fmt", ["bf16", "fp8"])
+def test_layer_with_drops_over_nan_memory(tokens, experts, top_k, fmt):
+    """Forward and backward with dropped routes give the same finite results
+    whatever the memory of their buffers held before."""
+    import mega_moe
+    from mega_moe.bench_configs import CaseSpec, make_inputs
+
+    inp = make_inputs(CaseSpec("drops", tokens, 512, 256, experts, top_k, "softmax_topk", True), device="cuda", seed=9,
+                      weight_scale=0.1)
+    sel = inp["selected"].clone()
+    sel[torch.rand(sel.shape, generator=torch.Generator().manual_seed(1)) < 0.1] = -1
+    names = ("grad_hidden", "grad_routing_weights", "grad_gate_up", "grad_fc2")
+    got = []
+    for fill in (0.0, float("nan")):
+        op = mega_moe.FusedMoEForward(None, max_tokens_per_rank=tokens, hidden_size=512, top_k=top_k,
+                                      num_experts=experts, config=mega_moe.MoEForwardConfig(save_fc1_dtype=fmt))
+        held = [torch.full((n,), fill, device="cuda") for n in [1 << 22] * 16 + [1 << 18] * 32 + [1 << 12] * 64 + [64] * 64]
+        del held  # the allocator hands this memory out again
+        out, saved = op.forward(inp["x"], sel, inp["gate_up"], inp["down"], inp["rw"], return_saved=True)
+        grads = mega_moe.moe_backward_triton(saved, inp["dy"])
+        got.append([out.clone()] + [grads[n].clone() for n in names])
+        del out, saved, grads, op
+    for name, a, b in zip(("out",) + names, *got):
+        assert bool(torch.isfinite(b).all()) and torch.equal(a, b), name

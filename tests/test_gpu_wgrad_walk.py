@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("E,n1,n2", [
     (1, 256, 256), (3, 512, 768),        # fewer experts than teams, few tiles
-    (5, 4096, 2048), (15, 1536, 2048),   # the same with several tiles per workgroup: one team
+    (1, 4096, 4096), (8, 2048, 2048),    # one team from one tile per workgroup on
+    (5, 4096, 2048), (15, 1536, 2048),   # the same with several tiles per workgroup
     (16, 256, 256), (17, 768, 768),      # 1 and 9 tiles per expert over 16-workgroup teams
     (40, 2048, 768),                     # 24 tiles: one and a half rounds per expert
 ])
